@@ -106,14 +106,6 @@ __device__ __forceinline__ void prioritise_long(bool long_running)
 
 constexpr int VA_LONG_ATTEMPTS = 160;  // ~2x the median attempts of an instance
 
-// Wait for this wave's outstanding vector-memory operations.  Placed at the end
-// of a refill, it retires the instance's parameter loads there; otherwise the
-// compiler cannot tell at the loop head whether a load is pending and waits
-// for every outstanding operation -- including the trajectory stores, which
-// count in the same in-order counter -- on each trip.  (gfx9 s_waitcnt
-// encoding: vmcnt 0, expcnt and lgkmcnt left at their maxima.)
-__device__ __forceinline__ void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
-
 template <int NN>
 __device__ __forceinline__ void exchange(double *slab, int lane, int gbase, double v,
                                          double (&out)[NN])

@@ -25,6 +25,14 @@ namespace va {
 enum { LANE_OK = 0, LANE_MAX_FAIL = 1, LANE_NONFINITE = 2, LANE_MAX_STEPS = 3 };
 enum { COST_REFERENCE = 0, COST_SUM = 1, COST_SQUARED_NORM = 2, COST_LINEAR = 3 };
 
+// Wait for this wave's outstanding vector-memory operations.  Placed at the end
+// of a refill, it retires the instance's parameter loads there; otherwise the
+// compiler cannot tell at the loop head whether a load is pending and waits
+// for every outstanding operation -- including the trajectory stores, which
+// count in the same in-order counter -- on each trip.  (gfx9 s_waitcnt
+// encoding: vmcnt 0, expcnt and lgkmcnt left at their maxima.)
+__device__ __forceinline__ void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+
 template <int N>
 __device__ __forceinline__ bool all_finite(const double *y)
 {
@@ -37,6 +45,14 @@ __device__ __forceinline__ bool all_finite(const double *y)
 // ---------------------------------------------------------------------------
 // Persistent forward
 // ---------------------------------------------------------------------------
+// What bounds it: one instance's chain of attempts where the batch leaves the
+// chip idle, the instructions of an attempt where it does not.  A lone wave pays 4
+// cycles for every instruction, so the loop holds one branch per attempt besides
+// the accept, and nothing in it waits for memory: a refill retires its loads
+// before the loop goes on (wait_vmem), and a step's row (t_n, h_n, y_n) is stored
+// whole when the step is accepted and h_n is known, two 16-byte stores for N = 2.
+// (With the waits on each step's stores and rows, here and in k_rev: solve of
+// Van der Pol, B=1024, 2.67 ms, oscillator, B=2^20, 49.2 ms; without 2.10 and 34.4.)
 template <class Sys, class Tab, bool Adaptive>
 __global__ void __launch_bounds__(256) k_fwd(FwdArgs a)
 {
@@ -52,10 +68,30 @@ __global__ void __launch_bounds__(256) k_fwd(FwdArgs a)
     double t = 0.0, dt = 0.0;
     int64_t b = 0;
     int32_t count = 0, rej = 0, tries = 0, st = LANE_OK;
-    bool new_step = true, have_k0 = false, need = true;
-    double *rows = nullptr;
+    bool need = true;
+    double *row = nullptr;  // row `count` of the instance
+
+    // The head of the controlled loop at the point (t, y): false when the instance
+    // is done (or has no room for another step), else dt clipped to end at t1.
+    auto begin_step = [&]() {
+        const bool more = Adaptive ? less_with_sign(t, sp.t1, dt)
+                                   : less_eq_with_sign(t + sp.dt0, sp.t1, sp.dt0);
+        if (more && count >= sp.cap) st = LANE_MAX_STEPS;
+        if constexpr (Adaptive)
+            if (less_with_sign(sp.t1, t + dt, dt)) dt = sp.t1 - t;
+        if constexpr (!Tab::FSAL) Sys::rhs(q, y, K[0]);
+        tries = 0;
+        return more && count < sp.cap;
+    };
+    auto store_row = [&](double h) {
+        row[0] = t;
+        row[1] = h;
+#pragma unroll
+        for (int i = 0; i < N; ++i) row[2 + i] = y[i];
+    };
 
     for (;;) {
+        bool finish = false;
         if (need) {
             b = atomicAdd(a.counter, 1);
             if (b >= B) break;
@@ -65,85 +101,46 @@ __global__ void __launch_bounds__(256) k_fwd(FwdArgs a)
             for (int i = 0; i < N; ++i) y[i] = a.y[(int64_t)i * B + b];
             t = sp.t0;
             dt = sp.dt0;
-            count = rej = tries = 0;
+            count = rej = 0;
             st = LANE_OK;
-            new_step = true;
-            have_k0 = false;
             need = false;
-            rows = a.traj + (size_t)b * (size_t)(sp.cap + 1) * F;
-        }
-        bool finish = false;
-        if (new_step) {
-            const bool more = Adaptive ? less_with_sign(t, sp.t1, dt)
-                                       : less_eq_with_sign(t + sp.dt0, sp.t1, sp.dt0);
-            if (!more) {
-                finish = true;
-            } else if (count >= sp.cap) {
-                st = LANE_MAX_STEPS;
-                finish = true;
-            } else {
-                double *r = rows + (size_t)count * F;
-                r[0] = t;
-#pragma unroll
-                for (int i = 0; i < N; ++i) r[2 + i] = y[i];
-                if (Adaptive && less_with_sign(sp.t1, t + dt, dt)) dt = sp.t1 - t;
-                if (!Tab::FSAL || !have_k0) {
-                    Sys::rhs(q, y, K[0]);
-                    have_k0 = true;
-                }
-                tries = 0;
-                new_step = false;
-            }
+            row = a.traj + (size_t)b * (size_t)(sp.cap + 1) * F;
+            wait_vmem();
+            if constexpr (Tab::FSAL) Sys::rhs(q, y, K[0]);
+            finish = !begin_step();
         }
         if (!finish) {
             const double h = Adaptive ? dt : sp.dt0;
             R::attempt(q, y, K, h, ynew, xerr);
+            bool accept = true, fail = false;
             if constexpr (Adaptive) {
                 const double err = R::error_norm(sp.atol, sp.rtol, h, y, K[0], xerr);
-                double dt_next;
-                const bool accept = control_step<Tab>(dt, err, dt_next);
-                if (!accept) {
-                    ++rej;
-                } else {
-                    const double tn = t + dt;
-                    rows[(size_t)count * F + 1] = stored_step(tn, t);
-                    t = tn;
-#pragma unroll
-                    for (int i = 0; i < N; ++i) y[i] = ynew[i];
-                    if constexpr (Tab::FSAL) {
-#pragma unroll
-                        for (int i = 0; i < N; ++i) K[0][i] = K[Tab::SF - 1][i];
-                    }
-                    ++count;
-                    new_step = true;
-                }
-                dt = dt_next;
-                ++tries;
-                if (tries > sp.max_attempts) {
-                    st = LANE_MAX_FAIL;
-                    finish = true;
-                }
-            } else {
-#pragma unroll
-                for (int i = 0; i < N; ++i) y[i] = ynew[i];
-                if constexpr (Tab::FSAL) {
-#pragma unroll
-                    for (int i = 0; i < N; ++i) K[0][i] = K[Tab::SF - 1][i];
-                }
+                accept = control_step<Tab>(h, err, dt);
+                fail = ++tries > sp.max_attempts;
+            }
+            if (accept) {
                 ++count;
-                const double tn = sp.t0 + (double)count * sp.dt0;
-                rows[(size_t)(count - 1) * F + 1] = stored_step(tn, t);
+                const double tn = Adaptive ? t + h : sp.t0 + (double)count * sp.dt0;
+                store_row(stored_step(tn, t));
+                row += F;
                 t = tn;
-                new_step = true;
+#pragma unroll
+                for (int i = 0; i < N; ++i) {
+                    y[i] = ynew[i];
+                    if constexpr (Tab::FSAL) K[0][i] = K[Tab::SF - 1][i];
+                }
+                finish = !begin_step();
+            } else {
+                ++rej;
+            }
+            if (fail) {
+                st = LANE_MAX_FAIL;
+                finish = true;
             }
         }
         if (finish) {
             if (st == LANE_OK) {
-                double *r = rows + (size_t)count * F;
-                r[0] = t;
-                r[1] = 0.0;
-#pragma unroll
-                for (int i = 0; i < N; ++i) r[2 + i] = y[i];
+                store_row(0.0);
                 if (!all_finite<N>(y)) st = LANE_NONFINITE;
             }
 #pragma unroll
@@ -238,6 +235,16 @@ __global__ void __launch_bounds__(256) k_rev(RevArgs a)
     int32_t o = 0, n = -1;
     bool need = true;
     const double *rows = nullptr;
+    // rows n and n - 1 of the sweep, each loaded two steps before its own, so that
+    // no step waits for memory (a step of a small system takes about 0.5 us, less
+    // than a read from HBM)
+    double h0 = 0.0, h1 = 0.0, y0[N] = {}, y1[N] = {};
+    auto load_row = [&](int32_t k, double &h, double (&y)[N]) {
+        const double *r = rows + (size_t)(k > 0 ? k : 0) * F;
+        h = r[1];
+#pragma unroll
+        for (int i = 0; i < N; ++i) y[i] = r[2 + i];
+    };
 
     for (;;) {
         if (need) {
@@ -268,11 +275,24 @@ __global__ void __launch_bounds__(256) k_rev(RevArgs a)
 #pragma unroll
             for (int k = 0; k < P; ++k) pbar[k] = 0.0;
             n = a.n_acc[b] - 1;
+            load_row(n, h0, y0);
+            load_row(n - 1, h1, y1);
             need = false;
+            wait_vmem();
         }
         if (n >= 0) {
-            const double *r = rows + (size_t)n * F;
-            back_prop_step<Sys, Tab>(q, r[1], r + 2, lam, pbar);
+            const double h = h0;
+            double y[N];
+            h0 = h1;
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                y[i] = y0[i];
+                y0[i] = y1[i];
+            }
+            load_row(n - 2, h1, y1);
+            // (the scheduler would move these loads to the end of the step)
+            __builtin_amdgcn_sched_barrier(0);
+            back_prop_step<Sys, Tab>(q, h, y, lam, pbar);
             --n;
         }
         if (n < 0) {
@@ -295,6 +315,9 @@ __global__ void __launch_bounds__(256) k_rev(RevArgs a)
 #pragma unroll
                 for (int k = 0; k < P; ++k) pbar[k] = 0.0;
                 n = a.n_acc[b] - 1;
+                load_row(n, h0, y0);
+                load_row(n - 1, h1, y1);
+                wait_vmem();
             }
         }
     }
