@@ -15,6 +15,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "va_pow.hpp"
 
 namespace va {
@@ -149,13 +151,14 @@ struct FivePow {
     }
 };
 
-// The controller pow's tables in LDS (5 KB per block): every kernel that runs the
+// The controller pow's tables in LDS (6 KB per block): every kernel that runs the
 // controller copies them in with load_ctrl_tables() at its start (a block-wide
 // barrier follows), so the two table reads on each attempt's dependent chain are
-// LDS reads instead of cache reads.
+// LDS reads instead of cache reads.  Entries lie on 16 bytes, so that each is
+// read by one 128-bit load (and a 64-bit one) at a constant offset.
 struct CtrlTablesLds {
-    double log[128][3];
-    uint64_t exp[256];
+    double2 log[128][2];  // (1/c, log c), (tail of log c, -)
+    ulonglong2 exp[128];  // (tail bits, scale bits)
 };
 
 __device__ __forceinline__ CtrlTablesLds &ctrl_lds()
@@ -168,9 +171,11 @@ __device__ __forceinline__ CtrlTablesLds &ctrl_lds()
 __device__ __forceinline__ void load_ctrl_tables()
 {
     CtrlTablesLds &t = ctrl_lds();
-    for (int k = threadIdx.x; k < 128 * 3; k += blockDim.x)
-        (&t.log[0][0])[k] = (&powtab::LOG[0][0])[k];
-    for (int k = threadIdx.x; k < 256; k += blockDim.x) t.exp[k] = powtab::EXP[k];
+    for (int k = threadIdx.x; k < 128; k += blockDim.x) {
+        t.log[k][0] = make_double2(powtab::LOG[k][0], powtab::LOG[k][1]);
+        t.log[k][1].x = powtab::LOG[k][2];
+        t.exp[k] = make_ulonglong2(powtab::EXP[2 * k], powtab::EXP[2 * k + 1]);
+    }
     __syncthreads();
 }
 
@@ -178,17 +183,91 @@ struct LdsTables {
     __device__ static void log_entry(int i, double &invc, double &logc, double &logctail)
     {
         const CtrlTablesLds &t = ctrl_lds();
-        invc = t.log[i][0];
-        logc = t.log[i][1];
-        logctail = t.log[i][2];
+        const double2 v = t.log[i][0];
+        invc = v.x;
+        logc = v.y;
+        logctail = t.log[i][1].x;
     }
-    __device__ static void exp_entry(uint64_t idx, uint64_t &tail_bits, uint64_t &scale_bits)
+    __device__ static void exp_entry(int i, uint64_t &tail_bits, uint64_t &scale_bits)
     {
-        const CtrlTablesLds &t = ctrl_lds();
-        tail_bits = t.exp[idx];
-        scale_bits = t.exp[idx + 1];
+        const ulonglong2 v = ctrl_lds().exp[i];
+        tail_bits = v.x;
+        scale_bits = v.y;
     }
 };
+
+// Constants as values in vector registers (Opaque: the compiler sees unknown
+// values formed once per kernel) or as literals, which it forms in scalar
+// registers at their uses, two scalar moves each.  A wave that has its SIMD to
+// itself pays those moves in full (every instruction issues in 4 cycles): the
+// kernels whose waves run alone keep the constants in registers.  With
+// several waves per SIMD the scalar moves issue beside other waves' vector
+// instructions, and the registers would cost occupancy.
+__device__ __forceinline__ double opaque(double x)
+{
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
+template <class Tab, bool Opaque>
+struct TabRegs {
+    double a[Tab::SF][Tab::SF], b[Tab::S], db[Tab::SF];
+    __device__ __forceinline__ TabRegs()
+    {
+#pragma unroll
+        for (int m = 0; m < Tab::SF; ++m)
+#pragma unroll
+            for (int j = 0; j < Tab::SF; ++j) {
+                a[m][j] = Tab::A[m][j];
+                if constexpr (Opaque)
+                    if (j < m && Tab::A[m][j] != 0.0) a[m][j] = opaque(a[m][j]);
+            }
+#pragma unroll
+        for (int j = 0; j < Tab::S; ++j) {
+            // an FSAL tableau's last stage input is the solution: the same values,
+            // so that the two sums stay one
+            b[j] = Tab::FSAL ? a[Tab::SF - 1][j] : Tab::B[j];
+            if constexpr (Opaque && !Tab::FSAL)
+                if (Tab::B[j] != 0.0) b[j] = opaque(b[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < Tab::SF; ++j) {
+            db[j] = Tab::HAS_ERR ? Tab::DB[j] : 0.0;
+            if constexpr (Opaque && Tab::HAS_ERR)
+                if (Tab::DB[j] != 0.0) db[j] = opaque(db[j]);
+        }
+    }
+};
+
+struct PowRegs {
+    double P0, P1, P2, P3, P4, P5, P6,
+        LN2_HI, LN2_LO, INV_LN2_128, NEG_LN2_HI_128, NEG_LN2_LO_128,
+        SHIFT, E2, E3, E4, E5;
+    __device__ __forceinline__ PowRegs()
+    {
+        using L = powref::PowLiterals;
+        P0 = opaque(L::P0);
+        P1 = opaque(L::P1);
+        P2 = opaque(L::P2);
+        P3 = opaque(L::P3);
+        P4 = opaque(L::P4);
+        P5 = opaque(L::P5);
+        P6 = opaque(L::P6);
+        LN2_HI = opaque(L::LN2_HI);
+        LN2_LO = opaque(L::LN2_LO);
+        INV_LN2_128 = opaque(L::INV_LN2_128);
+        NEG_LN2_HI_128 = opaque(L::NEG_LN2_HI_128);
+        NEG_LN2_LO_128 = opaque(L::NEG_LN2_LO_128);
+        SHIFT = opaque(L::SHIFT);
+        E2 = opaque(L::E2);
+        E3 = opaque(L::E3);
+        E4 = opaque(L::E4);
+        E5 = opaque(L::E5);
+    }
+};
+
+template <bool Opaque>
+using PowConsts = std::conditional_t<Opaque, PowRegs, powref::PowLiterals>;
 
 // Accept/reject decision and the next step size (default_step_adjuster with
 // max_dt = 0):
@@ -196,25 +275,28 @@ struct LdsTables {
 //   accept, err < 0.5:  h * (0.9 pow(max(5^-ORDER, err), -1/ORDER))
 //   accept otherwise:   h
 // One pow evaluation whose argument and exponent are selected per lane first,
-// so lanes of a wave that take different decisions share one instruction
-// stream (tables read through PowTables: LDS copies by default, which the
-// kernel must have loaded).  The exponents are the rounded quotients -1.0/q, as Boost forms them;
-// pow(5.0, -q) is 1/5^q exactly rounded, which the C library returns for the
-// orders here (q <= 8).
-template <class Tab, class PowTables = LdsTables>
-__device__ __forceinline__ bool control_step(double h, double err, double &h_next)
+// and selects instead of branches around it, so lanes of a wave that take
+// different decisions share one instruction stream (tables read through
+// PowTables: LDS copies by default, which the kernel must have loaded).  The
+// exponents are the rounded quotients -1.0/q, as Boost forms them; pow(5.0, -q)
+// is 1/5^q exactly rounded, which the C library returns for the orders here
+// (q <= 8).  A rejected step's err exceeds 1, so max(5^-q, err) is its argument as
+// well; arguments are cut at 1e300 (inf among them), where a rejected step's
+// factor is below 0.2 in any case.
+template <class Tab, class PowTables = LdsTables, class PC = powref::PowLiterals>
+__device__ __forceinline__ bool control_step(double h, double err, double &h_next,
+                                             const PC &pc = PC())
 {
     constexpr double lo = FivePow<Tab::ORDER>::inv();
     constexpr double y_inc = -1.0 / (double)Tab::ORDER;
     constexpr double y_dec = -1.0 / (double)(Tab::ERR_ORDER - 1);
     const bool accept = !(err > 1.0);
-    const double base = accept ? ((lo < err) ? err : lo) : err;
-    const double f = 0.9 * powref::pow_ctrl<PowTables>(base, accept ? y_inc : y_dec);
-    if (!accept) {
-        h_next = h * ((f < 0.2) ? 0.2 : f);
-    } else {
-        h_next = (err < 0.5) ? h * f : h;
-    }
+    double base = (lo < err) ? err : lo;
+    base = (base < 1e300) ? base : 1e300;
+    const double f = 0.9 * powref::pow_finite<PowTables>(base, accept ? y_inc : y_dec, pc);
+    const double cut = (f < 0.2) ? 0.2 : f;
+    const double grow = (err < 0.5) ? f : 1.0;
+    h_next = h * (accept ? grow : cut);
     return accept;
 }
 
@@ -386,33 +468,36 @@ struct ErrFirst {  // index of the first nonzero embedded-error weight
     }
 };
 
-template <class Sys, class Tab>
+template <class Sys, class Tab, bool Opaque = false>
 struct RK {
     static constexpr int N = Sys::N;
+    using Consts = TabRegs<Tab, Opaque>;
 
-    __device__ __forceinline__ static void stage_input(int m, double h, const double *y,
-                                                       const double (*K)[N], double *X)
+    __device__ __forceinline__ static void stage_input(const Consts &tc, int m, double h,
+                                                       const double *y, const double (*K)[N],
+                                                       double *X)
     {
 #pragma unroll
         for (int i = 0; i < N; ++i) X[i] = y[i];
 #pragma unroll
         for (int j = 0; j < Tab::SF; ++j) {
             if (j < m && Tab::A[m][j] != 0.0) {
-                const double ah = Tab::A[m][j] * h;
+                const double ah = tc.a[m][j] * h;
 #pragma unroll
                 for (int i = 0; i < N; ++i) X[i] = X[i] + ah * K[j][i];
             }
         }
     }
 
-    __device__ __forceinline__ static void attempt(const typename Sys::Params &q, const double *y,
+    __device__ __forceinline__ static void attempt(const Consts &tc,
+                                                   const typename Sys::Params &q, const double *y,
                                                    double (*K)[N], double h, double *ynew,
                                                    double *xerr)
     {
 #pragma unroll
         for (int m = 1; m < Tab::SF; ++m) {
             double X[N];
-            stage_input(m, h, y, K, X);
+            stage_input(tc, m, h, y, K, X);
             Sys::rhs(q, X, K[m]);
         }
 #pragma unroll
@@ -420,20 +505,20 @@ struct RK {
 #pragma unroll
         for (int j = 0; j < Tab::S; ++j) {
             if (Tab::B[j] != 0.0) {
-                const double bh = Tab::B[j] * h;
+                const double bh = tc.b[j] * h;
 #pragma unroll
                 for (int i = 0; i < N; ++i) ynew[i] = ynew[i] + bh * K[j][i];
             }
         }
         if constexpr (Tab::HAS_ERR) {
             constexpr int j0 = ErrFirst<Tab>::value();
-            const double d0 = Tab::DB[j0] * h;
+            const double d0 = tc.db[j0] * h;
 #pragma unroll
             for (int i = 0; i < N; ++i) xerr[i] = d0 * K[j0][i];
 #pragma unroll
             for (int j = j0 + 1; j < Tab::SF; ++j) {
                 if (Tab::DB[j] != 0.0) {
-                    const double dh = Tab::DB[j] * h;
+                    const double dh = tc.db[j] * h;
 #pragma unroll
                     for (int i = 0; i < N; ++i) xerr[i] = xerr[i] + dh * K[j][i];
                 }

@@ -273,38 +273,6 @@ __device__ __forceinline__ QueueRange queue_range(int64_t B, const int32_t *spli
     return q;
 }
 
-// The tableau's coefficients as values in registers.  With Opaque the compiler
-// sees them as unknown values formed once per kernel, so it keeps them in
-// vector registers instead of forming each 64-bit constant in scalar registers
-// on every use (two scalar moves each).  The values are the tableau's.
-template <class Tab, bool Opaque>
-struct TabRegs {
-    double a[Tab::SF][Tab::SF], b[Tab::S], db[Tab::SF];
-    __device__ __forceinline__ TabRegs()
-    {
-#pragma unroll
-        for (int m = 0; m < Tab::SF; ++m)
-#pragma unroll
-            for (int j = 0; j < Tab::SF; ++j) {
-                a[m][j] = Tab::A[m][j];
-                if constexpr (Opaque)
-                    if (j < m && Tab::A[m][j] != 0.0) asm volatile("" : "+v"(a[m][j]));
-            }
-#pragma unroll
-        for (int j = 0; j < Tab::S; ++j) {
-            b[j] = Tab::B[j];
-            if constexpr (Opaque)
-                if (Tab::B[j] != 0.0) asm volatile("" : "+v"(b[j]));
-        }
-#pragma unroll
-        for (int j = 0; j < Tab::SF; ++j) {
-            db[j] = Tab::HAS_ERR ? Tab::DB[j] : 0.0;
-            if constexpr (Opaque && Tab::HAS_ERR)
-                if (Tab::DB[j] != 0.0) asm volatile("" : "+v"(db[j]));
-        }
-    }
-};
-
 // ---------------------------------------------------------------------------
 // Forward sweep (persistent, refill per instance group)
 // ---------------------------------------------------------------------------

@@ -52,19 +52,24 @@ __device__ __forceinline__ bool all_finite(const double *y)
 // before the loop goes on (wait_vmem), and a step's row (t_n, h_n, y_n) is stored
 // whole when the step is accepted and h_n is known, two 16-byte stores for N = 2.
 // (With the waits on each step's stores and rows, here and in k_rev: solve of
-// Van der Pol, B=1024, 2.67 ms, oscillator, B=2^20, 49.2 ms; without 2.10 and 34.4.)
-template <class Sys, class Tab, bool Adaptive>
+// Van der Pol, B=1024, 2.67 ms, oscillator, B=2^20, 49.2 ms; without 2.10 and
+// 34.4; with selects in the step control and, for Lone, the constants in vector
+// registers 1.83 and 33.8.)
+template <class Sys, class Tab, bool Adaptive, bool Lone>
 __global__ void __launch_bounds__(256) k_fwd(FwdArgs a)
 {
     if constexpr (Adaptive) load_ctrl_tables();
     constexpr int N = Sys::N;
     constexpr int F = N + 2;  // row (t_n, h_n, y_n)
-    using R = RK<Sys, Tab>;
+    using R = RK<Sys, Tab, Lone>;
+    const TabRegs<Tab, Lone> tc;
+    const PowConsts<Lone && Adaptive> pc;
     const SolveParams sp = a.sp;
     const int64_t B = sp.B;
+    const int32_t cap = (int32_t)sp.cap;  // va_problem.max_steps
 
     typename Sys::Params q;
-    double y[N], K[Tab::SF][N], ynew[N], xerr[N];
+    double y[N], k0[N] = {};  // k0 = f(y)
     double t = 0.0, dt = 0.0;
     int64_t b = 0;
     int32_t count = 0, rej = 0, tries = 0, st = LANE_OK;
@@ -76,12 +81,12 @@ __global__ void __launch_bounds__(256) k_fwd(FwdArgs a)
     auto begin_step = [&]() {
         const bool more = Adaptive ? less_with_sign(t, sp.t1, dt)
                                    : less_eq_with_sign(t + sp.dt0, sp.t1, sp.dt0);
-        if (more && count >= sp.cap) st = LANE_MAX_STEPS;
+        if (more && count >= cap) st = LANE_MAX_STEPS;
         if constexpr (Adaptive)
             if (less_with_sign(sp.t1, t + dt, dt)) dt = sp.t1 - t;
-        if constexpr (!Tab::FSAL) Sys::rhs(q, y, K[0]);
+        if constexpr (!Tab::FSAL) Sys::rhs(q, y, k0);
         tries = 0;
-        return more && count < sp.cap;
+        return more && count < cap;
     };
     auto store_row = [&](double h) {
         row[0] = t;
@@ -106,16 +111,19 @@ __global__ void __launch_bounds__(256) k_fwd(FwdArgs a)
             need = false;
             row = a.traj + (size_t)b * (size_t)(sp.cap + 1) * F;
             wait_vmem();
-            if constexpr (Tab::FSAL) Sys::rhs(q, y, K[0]);
+            if constexpr (Tab::FSAL) Sys::rhs(q, y, k0);
             finish = !begin_step();
         }
         if (!finish) {
             const double h = Adaptive ? dt : sp.dt0;
-            R::attempt(q, y, K, h, ynew, xerr);
+            double K[Tab::SF][N], ynew[N], xerr[N];
+#pragma unroll
+            for (int i = 0; i < N; ++i) K[0][i] = k0[i];
+            R::attempt(tc, q, y, K, h, ynew, xerr);
             bool accept = true, fail = false;
             if constexpr (Adaptive) {
-                const double err = R::error_norm(sp.atol, sp.rtol, h, y, K[0], xerr);
-                accept = control_step<Tab>(h, err, dt);
+                const double err = R::error_norm(sp.atol, sp.rtol, h, y, k0, xerr);
+                accept = control_step<Tab>(h, err, dt, pc);
                 fail = ++tries > sp.max_attempts;
             }
             if (accept) {
@@ -127,7 +135,7 @@ __global__ void __launch_bounds__(256) k_fwd(FwdArgs a)
 #pragma unroll
                 for (int i = 0; i < N; ++i) {
                     y[i] = ynew[i];
-                    if constexpr (Tab::FSAL) K[0][i] = K[Tab::SF - 1][i];
+                    if constexpr (Tab::FSAL) k0[i] = K[Tab::SF - 1][i];
                 }
                 finish = !begin_step();
             } else {
@@ -157,22 +165,23 @@ __global__ void __launch_bounds__(256) k_fwd(FwdArgs a)
 // ---------------------------------------------------------------------------
 // Reverse step (detail/backpropagation.hpp:83-158) on one stored row pair.
 // ---------------------------------------------------------------------------
-template <class Sys, class Tab>
-__device__ __forceinline__ void back_prop_step(const typename Sys::Params &q, double h,
+template <class Sys, class Tab, bool Opaque>
+__device__ __forceinline__ void back_prop_step(const TabRegs<Tab, Opaque> &tc,
+                                               const typename Sys::Params &q, double h,
                                                const double *yn, double *lam, double *pbar)
 {
     // h = t_{n+1} - t_n as stored by the forward (the reference's GetDt).
     constexpr int N = Sys::N, S = Tab::S;
-    using R = RK<Sys, Tab>;
+    using R = RK<Sys, Tab, Opaque>;
     double K[Tab::SF][N], X[S][N], Kb[S][N];
 #pragma unroll
     for (int m = 0; m < S; ++m) {
-        R::stage_input(m, h, yn, K, X[m]);
+        R::stage_input(tc, m, h, yn, K, X[m]);
         Sys::rhs(q, X[m], K[m]);
     }
 #pragma unroll
     for (int m = 0; m < S; ++m) {
-        const double bh = Tab::B[m] * h;
+        const double bh = tc.b[m] * h;
 #pragma unroll
         for (int i = 0; i < N; ++i) Kb[m][i] = bh * lam[i];
     }
@@ -189,7 +198,7 @@ __device__ __forceinline__ void back_prop_step(const typename Sys::Params &q, do
         for (int j = 0; j < S; ++j) {
             if (j < m && Tab::A[m][j] != 0.0) {
 #pragma unroll
-                for (int i = 0; i < N; ++i) Kb[j][i] = Kb[j][i] + (xi[i] * Tab::A[m][j]) * h;
+                for (int i = 0; i < N; ++i) Kb[j][i] = Kb[j][i] + (xi[i] * tc.a[m][j]) * h;
             }
         }
     }
@@ -221,9 +230,10 @@ __device__ __forceinline__ double terminal_cost(int cost, const double *w, const
 // ---------------------------------------------------------------------------
 // Persistent reverse
 // ---------------------------------------------------------------------------
-template <class Sys, class Tab>
+template <class Sys, class Tab, bool Lone>
 __global__ void __launch_bounds__(256) k_rev(RevArgs a)
 {
+    const TabRegs<Tab, Lone> tc;
     constexpr int N = Sys::N, P = Sys::P, F = N + 2;
     const SolveParams sp = a.sp;
     const int64_t B = sp.B;
@@ -292,7 +302,7 @@ __global__ void __launch_bounds__(256) k_rev(RevArgs a)
             load_row(n - 2, h1, y1);
             // (the scheduler would move these loads to the end of the step)
             __builtin_amdgcn_sched_barrier(0);
-            back_prop_step<Sys, Tab>(q, h, y, lam, pbar);
+            back_prop_step<Sys>(tc, q, h, y, lam, pbar);
             --n;
         }
         if (n < 0) {
@@ -333,6 +343,7 @@ __global__ void __launch_bounds__(256) k_plain_fwd(PlainFwdArgs a)
     constexpr int N = Sys::N;
     constexpr int F = 2 + N;  // fields (t_n, h_n, y_n)
     using R = RK<Sys, Tab>;
+    const TabRegs<Tab, false> tc;
     const SolveParams sp = a.sp;
     const int64_t B = sp.B;
     const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -383,7 +394,7 @@ __global__ void __launch_bounds__(256) k_plain_fwd(PlainFwdArgs a)
     if constexpr (Adaptive) {
         int32_t tries = 0;
         for (;;) {
-            R::attempt(q, y, K, dt, ynew, xerr);
+            R::attempt(tc, q, y, K, dt, ynew, xerr);
             const double err = R::error_norm(sp.atol, sp.rtol, dt, y, K[0], xerr);
             double dt_next;
             const bool ok = control_step<Tab>(dt, err, dt_next);
@@ -411,7 +422,7 @@ __global__ void __launch_bounds__(256) k_plain_fwd(PlainFwdArgs a)
             if (ok) break;
         }
     } else {
-        R::attempt(q, y, K, sp.dt0, ynew, xerr);
+        R::attempt(tc, q, y, K, sp.dt0, ynew, xerr);
         const double tn = sp.t0 + (double)(step + 1) * sp.dt0;
         row[(size_t)B] = stored_step(tn, t);
         t = tn;
@@ -452,7 +463,7 @@ __global__ void __launch_bounds__(256) k_plain_rev(PlainRevArgs a)
     for (int i = 0; i < N; ++i) lam[i] = a.lambda[(int64_t)i * B + b];
 #pragma unroll
     for (int k = 0; k < P; ++k) pbar[k] = a.st.pbar[(int64_t)k * B + b];
-    back_prop_step<Sys, Tab>(q, h, yn, lam, pbar);
+    back_prop_step<Sys>(TabRegs<Tab, false>(), q, h, yn, lam, pbar);
 #pragma unroll
     for (int i = 0; i < N; ++i) a.lambda[(int64_t)i * B + b] = lam[i];
 #pragma unroll
@@ -462,16 +473,40 @@ __global__ void __launch_bounds__(256) k_plain_rev(PlainRevArgs a)
 // ---------------------------------------------------------------------------
 // Launchers and the dispatch table
 // ---------------------------------------------------------------------------
+// A launch whose waves have a SIMD each (at most one wave per SIMD of the 256
+// CUs): its time is the waves' own instruction count, and it takes the kernels
+// with the constants in vector registers.  Only small systems have them: the
+// state of a larger one needs the registers.
+constexpr int VA_LONE_THREADS = 256 * 4 * 64;
+
+template <class Sys>
+inline bool lone_waves(int grid, int block)
+{
+    return Sys::N <= 4 && (int64_t)grid * block <= VA_LONE_THREADS;
+}
+
 template <class Sys, class Tab, bool Ad>
 struct Launch {
     static hipError_t fwd(const FwdArgs &a, int grid, int block, hipStream_t s)
     {
-        hipLaunchKernelGGL((k_fwd<Sys, Tab, Ad>), dim3(grid), dim3(block), 0, s, a);
+        if constexpr (Sys::N <= 4) {
+            if (lone_waves<Sys>(grid, block)) {
+                hipLaunchKernelGGL((k_fwd<Sys, Tab, Ad, true>), dim3(grid), dim3(block), 0, s, a);
+                return hipGetLastError();
+            }
+        }
+        hipLaunchKernelGGL((k_fwd<Sys, Tab, Ad, false>), dim3(grid), dim3(block), 0, s, a);
         return hipGetLastError();
     }
     static hipError_t rev(const RevArgs &a, int grid, int block, hipStream_t s)
     {
-        hipLaunchKernelGGL((k_rev<Sys, Tab>), dim3(grid), dim3(block), 0, s, a);
+        if constexpr (Sys::N <= 4) {
+            if (lone_waves<Sys>(grid, block)) {
+                hipLaunchKernelGGL((k_rev<Sys, Tab, true>), dim3(grid), dim3(block), 0, s, a);
+                return hipGetLastError();
+            }
+        }
+        hipLaunchKernelGGL((k_rev<Sys, Tab, false>), dim3(grid), dim3(block), 0, s, a);
         return hipGetLastError();
     }
     static hipError_t pfwd(const PlainFwdArgs &a, int grid, int block, hipStream_t s)
@@ -487,7 +522,7 @@ struct Launch {
     static int occ_fwd(int block)
     {
         int nb = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_fwd<Sys, Tab, Ad>, block, 0) !=
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_fwd<Sys, Tab, Ad, false>, block, 0) !=
             hipSuccess)
             return 1;
         return nb;
@@ -495,7 +530,7 @@ struct Launch {
     static int occ_rev(int block)
     {
         int nb = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_rev<Sys, Tab>, block, 0) !=
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_rev<Sys, Tab, false>, block, 0) !=
             hipSuccess)
             return 1;
         return nb;

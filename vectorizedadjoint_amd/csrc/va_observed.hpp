@@ -74,6 +74,7 @@ __global__ void __launch_bounds__(256) k_obs_fwd(ObsFwdArgs a)
     constexpr int N = Sys::N;
     constexpr int F = N + 2, FC = N + 3;
     using R = RK<Sys, Tab>;
+    const TabRegs<Tab, false> tc;
     const SolveParams sp = a.sp;
     const int64_t B = sp.B;
     const int K = a.K;
@@ -196,7 +197,7 @@ __global__ void __launch_bounds__(256) k_obs_fwd(ObsFwdArgs a)
         }
         if (!finish) {
             const double h = dt;
-            R::attempt(q, y, Kst, h, ynew, xerr);
+            R::attempt(tc, q, y, Kst, h, ynew, xerr);
             const double err = R::error_norm(sp.atol, sp.rtol, h, y, Kst[0], xerr);
             double dt_next;
             if (!control_step<Tab>(dt, err, dt_next)) {
@@ -269,6 +270,7 @@ __device__ void recompute_segment(const typename Sys::Params &q, const SolvePara
 {
     constexpr int N = Sys::N, FS = N + 1, FC = N + 3;
     using R = RK<Sys, Tab>;
+    const TabRegs<Tab, false> tc;
     double y[N], Kst[Tab::SF][N], ynew[N], xerr[N];
     double t = c[0], dt = c[1], dt_keep = 0.0;
     int kobs = (int)c[2];
@@ -315,7 +317,7 @@ __device__ void recompute_segment(const typename Sys::Params &q, const SolvePara
             new_step = false;
         }
         const double h = dt;
-        R::attempt(q, y, Kst, h, ynew, xerr);
+        R::attempt(tc, q, y, Kst, h, ynew, xerr);
         const double err = R::error_norm(sp.atol, sp.rtol, h, y, Kst[0], xerr);
         double dt_next;
         const bool ok = control_step<Tab>(dt, err, dt_next);
@@ -567,7 +569,7 @@ __device__ void obs_rev_backward(const ObsRevArgs &a, ObsPipe &Pp, int pair, int
 #pragma unroll
                     for (int i = 0; i < N; ++i) yk[i] = yn[i];
                     if (k > 0) load_row(k - 1);
-                    back_prop_step<Sys, Tab>(q, hk, yk, lam, pbar);
+                    back_prop_step<Sys>(TabRegs<Tab, false>(), q, hk, yk, lam, pbar);
                     kobs = obs_jumps<N>(orow, a.obs_y, kobs, onext, n0 + k, yk, lam);
                 }
                 if (ij == 0) finish(ib);
@@ -641,7 +643,7 @@ __global__ void __launch_bounds__(256) k_obs_rev(ObsRevArgs a)
             const double *rows = a.st.traj + (size_t)b * (size_t)(sp.cap + 1) * F;
             for (int32_t n = cnt - 1; n >= 0; --n) {
                 const double *r = rows + (size_t)n * F;
-                back_prop_step<Sys, Tab>(q, r[1], r + 2, lam, pbar);
+                back_prop_step<Sys>(TabRegs<Tab, false>(), q, r[1], r + 2, lam, pbar);
                 kobs = obs_jumps<N>(orow, a.obs_y, kobs, onext, n, r + 2, lam);
             }
         } else {
@@ -667,7 +669,7 @@ __global__ void __launch_bounds__(256) k_obs_rev(ObsRevArgs a)
 #pragma unroll
                     for (int i = 0; i < N; ++i) yk[i] = yn[i];
                     if (k > 0) load_row(k - 1);
-                    back_prop_step<Sys, Tab>(q, hk, yk, lam, pbar);
+                    back_prop_step<Sys>(TabRegs<Tab, false>(), q, hk, yk, lam, pbar);
                     kobs = obs_jumps<N>(orow, a.obs_y, kobs, onext, n0 + k, yk, lam);
                 }
             };

@@ -51,26 +51,42 @@ namespace powref {
 VA_POW_HD double as_double(uint64_t u) { return __builtin_bit_cast(double, u); }
 VA_POW_HD uint64_t as_bits(double d) { return __builtin_bit_cast(uint64_t, d); }
 
-// log1p polynomial, scaled by the evaluation (p0 = -1/2)
-constexpr double P0 = -0x1p-1;
-constexpr double P1 = 0x1.555555555556p-2 * -2;
-constexpr double P2 = -0x1.0000000000006p-2 * -2;
-constexpr double P3 = 0x1.999999959554ep-3 * 4;
-constexpr double P4 = -0x1.555555529a47ap-3 * 4;
-constexpr double P5 = 0x1.2495b9b4845e9p-3 * -8;
-constexpr double P6 = -0x1.0002b8b263fc3p-3 * -8;
-constexpr double LN2_HI = 0x1.62e42fefa3800p-1;
-constexpr double LN2_LO = 0x1.ef35793c76730p-45;
-// exp: 128/ln2, -ln2/128 split, rounding shift, polynomial
-constexpr double INV_LN2_128 = 0x1.71547652b82fep0 * 128;
-constexpr double NEG_LN2_HI_128 = -0x1.62e42fefa0000p-8;
-constexpr double NEG_LN2_LO_128 = -0x1.cf79abc9e3b3ap-47;
-constexpr double SHIFT = 0x1.8p52;
-constexpr double E2 = 0x1.ffffffffffdbdp-2;
-constexpr double E3 = 0x1.555555555543cp-3;
-constexpr double E4 = 0x1.55555cf172b91p-5;
-constexpr double E5 = 0x1.1111167a4d017p-7;
-constexpr uint64_t OFF = 0x3fe6955500000000ull;
+// a double from its halves (two moves on the device, no 64-bit arithmetic)
+struct Halves {
+    uint32_t lo, hi;
+};
+VA_POW_HD double from_halves(uint32_t hi, uint32_t lo)
+{
+    return __builtin_bit_cast(double, Halves{lo, hi});
+}
+
+// The algorithm's constants, as literals: each use forms the 64-bit value in a
+// scalar register pair.  A caller may pass an object with the same members
+// instead (CtrlRegs in va_device.hpp keeps them in vector registers).
+struct PowLiterals {
+    // log1p polynomial, scaled by the evaluation (p0 = -1/2)
+    static constexpr double P0 = -0x1p-1;
+    static constexpr double P1 = 0x1.555555555556p-2 * -2;
+    static constexpr double P2 = -0x1.0000000000006p-2 * -2;
+    static constexpr double P3 = 0x1.999999959554ep-3 * 4;
+    static constexpr double P4 = -0x1.555555529a47ap-3 * 4;
+    static constexpr double P5 = 0x1.2495b9b4845e9p-3 * -8;
+    static constexpr double P6 = -0x1.0002b8b263fc3p-3 * -8;
+    static constexpr double LN2_HI = 0x1.62e42fefa3800p-1;
+    static constexpr double LN2_LO = 0x1.ef35793c76730p-45;
+    // exp: 128/ln2, -ln2/128 split, rounding shift, polynomial
+    static constexpr double INV_LN2_128 = 0x1.71547652b82fep0 * 128;
+    static constexpr double NEG_LN2_HI_128 = -0x1.62e42fefa0000p-8;
+    static constexpr double NEG_LN2_LO_128 = -0x1.cf79abc9e3b3ap-47;
+    static constexpr double SHIFT = 0x1.8p52;
+    static constexpr double E2 = 0x1.ffffffffffdbdp-2;
+    static constexpr double E3 = 0x1.555555555543cp-3;
+    static constexpr double E4 = 0x1.55555cf172b91p-5;
+    static constexpr double E5 = 0x1.1111167a4d017p-7;
+};
+// bits of 0x1.69555p-1, below which the scaled argument z does not lie; their low
+// half is zero, so the argument reduction works on the high 32 bits
+constexpr uint32_t OFF_HI = 0x3fe69555u;
 
 // Table access.  GlobalTables reads the constant tables; a caller may supply
 // another accessor with the same two functions (the kernels read LDS copies).
@@ -81,36 +97,37 @@ struct GlobalTables {
         logc = powtab::LOG[i][1];
         logctail = powtab::LOG[i][2];
     }
-    VA_POW_HD static void exp_entry(uint64_t idx, uint64_t &tail_bits, uint64_t &scale_bits)
+    VA_POW_HD static void exp_entry(int i, uint64_t &tail_bits, uint64_t &scale_bits)
     {
-        tail_bits = powtab::EXP[idx];
-        scale_bits = powtab::EXP[idx + 1];
+        tail_bits = powtab::EXP[2 * i];
+        scale_bits = powtab::EXP[2 * i + 1];
     }
 };
 
 // log(x) as hi + *lo for x > 0 normal (x given by its bits)
-template <class T = GlobalTables>
-VA_POW_HD double log_hilo(uint64_t ix, double *lo)
+template <class T = GlobalTables, class C = PowLiterals>
+VA_POW_HD double log_hilo(uint64_t ix, double *lo, const C &c = C())
 {
-    const uint64_t tmp = ix - OFF;
-    const int i = (int)((tmp >> 45) & 127);
-    const int k = (int)((int64_t)tmp >> 52);
-    const double z = as_double(ix - (tmp & (0xfffull << 52)));
+    const uint32_t hx = (uint32_t)(ix >> 32), tmp = hx - OFF_HI;
+    const int i = (int)((tmp >> 13) & 127);
+    const int k = (int)tmp >> 20;
+    const double z = from_halves(hx - (tmp & 0xfff00000u), (uint32_t)ix);
     const double kd = (double)k;
     double invc, logc, logctail;
     T::log_entry(i, invc, logc, logctail);
     const double r = fma(z, invc, -1.0);
-    const double t1 = fma(kd, LN2_HI, logc);
+    const double t1 = fma(kd, c.LN2_HI, logc);
     const double t2 = t1 + r;
-    const double lo1 = fma(kd, LN2_LO, logctail);
+    const double lo1 = fma(kd, c.LN2_LO, logctail);
     const double lo2 = t1 - t2 + r;
-    const double ar = P0 * r;
+    const double ar = c.P0 * r;
     const double ar2 = r * ar;
     const double ar3 = r * ar2;
     const double hi = t2 + ar2;
     const double lo3 = fma(ar, r, -ar2);
     const double lo4 = t2 - hi + ar2;
-    const double q = fma(ar2, fma(ar2, fma(r, P6, P5), fma(r, P4, P3)), fma(r, P2, P1));
+    const double q =
+        fma(ar2, fma(ar2, fma(r, c.P6, c.P5), fma(r, c.P4, c.P3)), fma(r, c.P2, c.P1));
     const double l = fma(ar3, q, lo1 + lo2 + lo3 + lo4);
     const double y = hi + l;
     *lo = hi - y + l;
@@ -118,36 +135,42 @@ VA_POW_HD double log_hilo(uint64_t ix, double *lo)
 }
 
 // exp(x + xtail) for |x| in [2^-54, 512)
-template <class T = GlobalTables>
-VA_POW_HD double exp_hilo(double x, double xtail)
+template <class T = GlobalTables, class C = PowLiterals>
+VA_POW_HD double exp_hilo(double x, double xtail, const C &c = C())
 {
-    double kd = fma(INV_LN2_128, x, SHIFT);
-    const uint64_t ki = as_bits(kd);
-    kd = kd - SHIFT;
-    double r = fma(kd, NEG_LN2_LO_128, fma(kd, NEG_LN2_HI_128, x));
+    double kd = fma(c.INV_LN2_128, x, c.SHIFT);
+    const uint32_t ki = (uint32_t)as_bits(kd);
+    kd = kd - c.SHIFT;
+    double r = fma(kd, c.NEG_LN2_LO_128, fma(kd, c.NEG_LN2_HI_128, x));
     r = r + xtail;
-    const uint64_t idx = 2 * (ki & 127);
-    const uint64_t top = ki << 45;
     uint64_t tail_bits, scale_bits;
-    T::exp_entry(idx, tail_bits, scale_bits);
+    T::exp_entry((int)(ki & 127), tail_bits, scale_bits);
     const double tail = as_double(tail_bits);
-    const uint64_t sbits = scale_bits + top;
+    // scale = 2^(ki / 128): the table's entry with ki / 128 added to its exponent
+    // (ki << 45 in the 64-bit value: the high half alone)
     const double r2 = r * r;
-    const double tmp = fma(r2 * r2, fma(r, E5, E4), fma(r2, fma(r, E3, E2), tail + r));
-    const double scale = as_double(sbits);
+    const double tmp = fma(r2 * r2, fma(r, c.E5, c.E4), fma(r2, fma(r, c.E3, c.E2), tail + r));
+    const double scale =
+        from_halves((uint32_t)(scale_bits >> 32) + (ki << 13), (uint32_t)scale_bits);
     return fma(scale, tmp, scale);
 }
 
-// pow(x, y) on the domain stated above
+// pow(x, y) on the domain stated above, x finite
+template <class T = GlobalTables, class C = PowLiterals>
+VA_POW_HD double pow_finite(double x, double y, const C &c = C())
+{
+    double lo;
+    const double hi = log_hilo<T>(as_bits(x), &lo, c);
+    const double ehi = y * hi;
+    const double elo = fma(y, lo, fma(y, hi, -ehi));
+    return exp_hilo<T>(ehi, elo, c);
+}
+
 template <class T = GlobalTables>
 VA_POW_HD double pow_ctrl(double x, double y)
 {
     if (x == __builtin_huge_val()) return 0.0;
-    double lo;
-    const double hi = log_hilo<T>(as_bits(x), &lo);
-    const double ehi = y * hi;
-    const double elo = fma(y, lo, fma(y, hi, -ehi));
-    return exp_hilo<T>(ehi, elo);
+    return pow_finite<T>(x, y);
 }
 
 }  // namespace powref
