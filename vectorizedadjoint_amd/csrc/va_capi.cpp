@@ -529,11 +529,11 @@ bool split_solve(const va_handle *h)
 // smaller share speeds up the long instances less than it slows down the
 // bulk.  Room for both waves of each of the solve's long-instance blocks made
 // the bulk's reverse 9% slower.)
-int bulk_grid(const va_handle *h, int64_t lanes)
+int bulk_grid(const va_handle *h, int64_t lanes, int parts = 1)
 {
     const int per_block = h->ks.slots(h->block);
     const int reserve = blocks_for((int64_t)VA_LONG_MAX * h->ks.slots(64), per_block);
-    const int g = blocks_for(std::min<int64_t>(lanes, h->pb.batch), per_block);
+    const int g = blocks_for(std::min<int64_t>(lanes, h->pb.batch * parts), per_block);
     return std::max(1, g - reserve);
 }
 
@@ -665,9 +665,24 @@ va_status forward_persistent(va_handle *h, double *y, const double *p, hipStream
     return VA_OK;
 }
 
+// Seeds a work item of a reverse of nout seeds takes.  The Lotka-Volterra groups
+// recompute the stages for every seed either way, so each seed is an item of its
+// own and the chip has nout times the chains to run side by side (N=5, B=8192,
+// five seeds: reverse 410 us with each instance's seeds in turn).  A lane with an
+// instance of its own can take two seeds through one sweep; while every seed still
+// finds a SIMD slot alone (one wave per SIMD), separate lanes are shorter chains.
+// Items are counted in 32 bits: a batch with more takes all seeds in turn.
+int32_t seeds_per_item(const va_handle *h, int nout)
+{
+    if (nout <= 1 || h->ks.table_version < 2 || h->pb.batch > (int64_t)(1 << 30) / nout) return 0;
+    if (h->ks.layout == 1) return 1;
+    return h->pb.batch * nout <= (int64_t)h->cu_count * 4 * 64 ? 1 : 2;
+}
+
+// identity: the seeds are the unit vectors (lambda is not used, mu = 0.0 + sum).
 va_status reverse_persistent(va_handle *h, const double *p, int cost, const double *cost_w,
                              const double *yT, double *J, double *lambda, double *mu, int nout,
-                             hipStream_t s)
+                             hipStream_t s, bool identity = false)
 {
     const int64_t B = h->pb.batch;
     va_status st = fill_i32(h->counters + 1, 0, 1, s);
@@ -691,19 +706,23 @@ va_status reverse_persistent(va_handle *h, const double *p, int cost, const doub
     a.mu = mu;
     a.nout = nout;
     a.counter = h->counters + 1;
+    a.seeds_per_item = cost ? 0 : seeds_per_item(h, nout);
+    a.identity = identity ? 1 : 0;
     const bool im = instance_major(h);
+    const bool add = cost == 0 && !identity;
     const int nseed = cost ? 1 : nout;
+    const int parts = va::rev_items(a).parts;
     if (split) {
         a.split = h->counters + h->nlong_idx;
         a.part = 1;
         if ((st = fork_side(h, s))) return st;
         // one seed: a block of three waves per long instance, as in a solve
         if (nseed == 1) VA_HIP(h->ks.long_rev(a, VA_LONG_MAX, 192, s));
-        else VA_HIP(h->ks.long_rev(a, VA_LONG_MAX / 4, 256, s));
+        else VA_HIP(h->ks.long_rev(a, VA_LONG_MAX * parts / 4, 256, s));
         va::RevArgs ab = a;
         if (im && (st = bulk_instance_major(h, p, &ab, nseed, h->side))) return st;
-        VA_HIP(h->ks.rev(ab, bulk_grid(h, h->lanes_rev), h->block, h->side));
-        if (im && (st = pbar_to_mu(h, mu, nseed, cost == 0, h->side, h->pbar_set))) return st;
+        VA_HIP(h->ks.rev(ab, bulk_grid(h, h->lanes_rev, parts), h->block, h->side));
+        if (im && (st = pbar_to_mu(h, mu, nseed, add, h->side, h->pbar_set))) return st;
         return join_side(h, s);
     }
     if (im) {
@@ -711,9 +730,9 @@ va_status reverse_persistent(va_handle *h, const double *p, int cost, const doub
         a.p = h->pim;
         if ((st = pbar_instance_major(h, a, nseed))) return st;
     }
-    const int64_t lanes = std::min<int64_t>(h->lanes_rev, B);
+    const int64_t lanes = std::min<int64_t>(h->lanes_rev, B * parts);
     VA_HIP(h->ks.rev(a, blocks_for(lanes, h->ks.slots(h->block)), h->block, s));
-    if (im) return pbar_to_mu(h, mu, nseed, cost == 0, s);
+    if (im) return pbar_to_mu(h, mu, nseed, add, s);
     return VA_OK;
 }
 
@@ -961,12 +980,14 @@ va_status check_problem(const va_problem *pb, va::KernelSet *ks_out,
         if (pb->system != VA_SYSTEM_USER)
             return fail(VA_ERR_INVALID, "a kernel table needs system VA_SYSTEM_USER");
         if (given->table_size != (int32_t)sizeof(va::KernelSet) ||
-            given->table_version != va::VA_KERNEL_TABLE_VERSION || !given->fwd || !given->rev)
+            given->table_version < va::VA_KERNEL_TABLE_OLDEST ||
+            given->table_version > va::VA_KERNEL_TABLE_VERSION || !given->fwd || !given->rev)
             return fail(VA_ERR_INVALID,
                         "kernel table of size %d, version %d: this library takes size %d, "
-                        "version %d (rebuild the system's translation unit against its headers)",
+                        "versions %d to %d (rebuild the system's translation unit against its "
+                        "headers)",
                         given->table_size, given->table_version, (int)sizeof(va::KernelSet),
-                        va::VA_KERNEL_TABLE_VERSION);
+                        va::VA_KERNEL_TABLE_OLDEST, va::VA_KERNEL_TABLE_VERSION);
         if (given->n != pb->n_state)
             return fail(VA_ERR_INVALID, "the kernel table is for N=%d, the problem says %d",
                         given->n, pb->n_state);
@@ -1325,6 +1346,12 @@ va_status va_sensitivity_matrix(va_handle *h, const double *p, double *S, void *
     hipStream_t s = (hipStream_t)stream;
     const int64_t B = h->pb.batch;
     const int n = h->ks.n, np = h->ks.np;
+    if (h->pb.mode == VA_MODE_PERSISTENT && h->ks.table_version >= 2) {
+        // the kernels form the unit seeds and write S whole
+        if (!h->have_forward)
+            return fail(VA_ERR_STATE, "va_adjoint needs a va_forward first");
+        return reverse_persistent(h, p, 0, nullptr, nullptr, nullptr, nullptr, S, n, s, true);
+    }
     double *lam = nullptr;
     VA_HIP(hipMallocAsync((void **)&lam, sizeof(double) * (size_t)n * n * B, s));
     hipLaunchKernelGGL(k_identity_seeds, dim3(blocks_for((int64_t)n * n * B, 256)), dim3(256), 0,

@@ -228,7 +228,7 @@ __device__ __forceinline__ void put_pbar(const RevArgs &a, int64_t o, int64_t k,
         a.mu[(o * a.sp.B + b) * P + k] = x;
     } else {
         double *m = a.mu + (o * P + k) * a.sp.B + b;
-        *m = a.cost ? 0.0 + x : *m + x;
+        *m = a.cost || a.identity ? 0.0 + x : *m + x;
     }
 }
 
@@ -720,7 +720,7 @@ __global__ void __launch_bounds__(256) k_glv_rows2_fwd(FwdArgs a)
 // the same operations in the same order as in the oracle.
 // ---------------------------------------------------------------------------
 template <int NN, class Tab, bool OneShot>
-__device__ __forceinline__ void glv_rows_rev_body(const RevArgs &a, int64_t one)
+__device__ __forceinline__ void glv_rows_rev_body(const RevArgs &a, int64_t one, int32_t one_seed)
 {
     using L = GlvRows<NN>;
     constexpr int F = L::F, S = Tab::S, P = NN + NN * NN;
@@ -749,12 +749,27 @@ __device__ __forceinline__ void glv_rows_rev_body(const RevArgs &a, int64_t one)
     // row nr's (h, y_i) of this lane, loaded one iteration ahead of its use
     double h_nxt = 0.0, y_nxt = 0.0, h_back = 0.0;
     int64_t b = 0;
-    int32_t o = 0, nr = -1;
+    int32_t o = 0, o_end = 0, nr = -1;
     int par = 0;  // slot parity of the step being reversed
     bool need = true, back = false, taken = false;
     const double *rows = nullptr;
     double v[NN];
     const QueueRange q = queue_range(B, a.split, a.part);
+    const RevItems items = rev_items(a);
+    // the seed o of the instance: its lambda, cleared sums, its last row
+    auto start_sweep = [&]() {
+        if (!a.cost)
+            lam = a.identity ? (o == i ? 1.0 : 0.0) : a.lambda[((int64_t)o * NN + i) * B + b];
+        rbar = 0.0;
+#pragma unroll
+        for (int j = 0; j < NN; ++j) Abar[j] = 0.0;
+        nr = a.n_acc[b] - 1;
+        if (nr >= 0) {
+            h_nxt = rows[(size_t)nr * F + 1];
+            y_nxt = rows[(size_t)nr * F + 2 + i];
+        }
+        wait_vmem();
+    };
 
     for (;;) {
         if constexpr (OneShot) __builtin_amdgcn_s_setprio(3);
@@ -764,18 +779,27 @@ __device__ __forceinline__ void glv_rows_rev_body(const RevArgs &a, int64_t one)
                 if (taken) break;
                 taken = true;
                 b = one;
+                o = one_seed;
             } else {
                 if (i == 0) gidx[wv][grp] = atomicAdd(a.counter, 1);
                 __builtin_amdgcn_wave_barrier();
-                b = q.lo + gidx[wv][grp];
+                const int32_t k = gidx[wv][grp];
                 __builtin_amdgcn_wave_barrier();
+                o = 0;
+                if (items.parts > 1) {
+                    const int32_t pos = k / items.parts;
+                    o = (k - pos * items.parts) * items.per;
+                    b = q.lo + pos;
+                } else {
+                    b = q.lo + k;
+                }
                 if (b >= q.hi) break;
                 if (a.order) b = a.order[b];
             }
+            o_end = o + items.per < items.seeds ? o + items.per : items.seeds;
             if (a.status[b] != LANE_OK) {
-                const int nseed = a.cost ? 1 : a.nout;
-                for (int oo = 0; oo < nseed; ++oo) {
-                    a.lambda[((int64_t)oo * NN + i) * B + b] = qnan;
+                for (int oo = o; oo < o_end; ++oo) {
+                    if (!a.identity) a.lambda[((int64_t)oo * NN + i) * B + b] = qnan;
                     put_pbar_nan<NN, !OneShot>(a, oo, i, b);
                     for (int j = 0; j < NN; ++j)
                         put_pbar_nan<NN, !OneShot>(a, oo, NN * (i + 1) + j, b);
@@ -791,7 +815,6 @@ __device__ __forceinline__ void glv_rows_rev_body(const RevArgs &a, int64_t one)
                 Acol[j] = param<NN, !OneShot>(a, NN * (j + 1) + i, b);
             }
             rows = a.traj + (size_t)b * (size_t)(sp.cap + 1) * F;
-            o = 0;
             if (a.cost) {
                 const double yT = a.yT[(int64_t)i * B + b];
                 // terminal cost: J = fold over i in order, lambda_i from y_i(T)
@@ -807,20 +830,10 @@ __device__ __forceinline__ void glv_rows_rev_body(const RevArgs &a, int64_t one)
                 else if (a.cost == COST_SQUARED_NORM) lam = 2.0 * yT;
                 else lam = a.cost_w[i];
                 if (i == 0) a.J[b] = J;
-            } else {
-                lam = a.lambda[(int64_t)i * B + b];
             }
-            rbar = 0.0;
-#pragma unroll
-            for (int j = 0; j < NN; ++j) Abar[j] = 0.0;
-            nr = a.n_acc[b] - 1;
+            start_sweep();
             back = false;
-            if (nr >= 0) {
-                h_nxt = rows[(size_t)nr * F + 1];
-                y_nxt = rows[(size_t)nr * F + 2 + i];
-            }
             need = false;
-            wait_vmem();
         }
         if (nr >= 0 || back) {
             // recompute step nr (stage inputs from (h_nr, y_nr), backpropagation.hpp:24-64)
@@ -904,27 +917,14 @@ __device__ __forceinline__ void glv_rows_rev_body(const RevArgs &a, int64_t one)
             --nr;
         }
         if (!back) {
-            const int64_t lo = (int64_t)o * NN;
-            a.lambda[(lo + i) * B + b] = lam;
+            if (!a.identity) a.lambda[((int64_t)o * NN + i) * B + b] = lam;
             put_pbar<NN, !OneShot>(a, o, i, b, rbar);
 #pragma unroll
             for (int k = 0; k < NN; ++k) put_pbar<NN, !OneShot>(a, o, NN * (k + 1) + i, b, Abar[k]);
             if (!OneShot && a.pbar_set && i == 0) a.pbar_set[b] = 1;
             ++o;
-            if (a.cost || o >= a.nout) {
-                need = true;
-            } else {
-                lam = a.lambda[((int64_t)o * NN + i) * B + b];
-                rbar = 0.0;
-#pragma unroll
-                for (int j = 0; j < NN; ++j) Abar[j] = 0.0;
-                nr = a.n_acc[b] - 1;
-                if (nr >= 0) {
-                    h_nxt = rows[(size_t)nr * F + 1];
-                    y_nxt = rows[(size_t)nr * F + 2 + i];
-                }
-                wait_vmem();
-            }
+            need = o >= o_end;
+            if (!need) start_sweep();
         }
     }
 }
@@ -932,7 +932,7 @@ __device__ __forceinline__ void glv_rows_rev_body(const RevArgs &a, int64_t one)
 template <int NN, class Tab>
 __global__ void __launch_bounds__(256) k_glv_rows_rev(RevArgs a)
 {
-    glv_rows_rev_body<NN, Tab, false>(a, 0);
+    glv_rows_rev_body<NN, Tab, false>(a, 0, 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1255,9 +1255,12 @@ __global__ void __launch_bounds__(192) k_glv_rows_long_adj(RevArgs ra)
 template <int NN, class Tab>
 __global__ void __launch_bounds__(256) k_glv_rows_long_rev(RevArgs ra)
 {
-    const int64_t w = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (w >= *ra.split || w >= ra.sp.B) return;
-    glv_rows_rev_body<NN, Tab, true>(ra, ra.order[w]);
+    // a wave per (instance, group of seeds)
+    const int32_t w = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    const RevItems items = rev_items(ra);
+    const int32_t pos = w / items.parts;
+    if (pos >= *ra.split || pos >= ra.sp.B) return;
+    glv_rows_rev_body<NN, Tab, true>(ra, ra.order[pos], (w - pos * items.parts) * items.per);
 }
 
 // ---------------------------------------------------------------------------

@@ -53,7 +53,26 @@ struct RevArgs {
     const int32_t *split = nullptr;  // as in FwdArgs
     int32_t part = 0;
     int32_t *pbar_set = nullptr;     // [B] or null
+    // (cost == 0) seeds that one work item takes: 0 all of them, else items are
+    // (instance, group of so many seeds) pairs.  See seeds_per_item() in va_capi.cpp.
+    int32_t seeds_per_item = 0;
+    // (cost == 0) the seeds are the unit vectors (nout = N): lambda is neither read
+    // nor written, and mu = 0.0 + sum
+    int32_t identity = 0;
 };
+
+// The work items of a reverse: groups of seeds per instance.
+struct RevItems {
+    int32_t seeds, per, parts;
+};
+__host__ __device__ inline RevItems rev_items(const RevArgs &a)
+{
+    RevItems r;
+    r.seeds = a.cost ? 1 : a.nout;
+    r.per = a.seeds_per_item > 0 ? a.seeds_per_item : r.seeds;
+    r.parts = (r.seeds + r.per - 1) / r.per;
+    return r;
+}
 
 // Plain form: one launch per accepted step, state in HBM, no refill, full
 // trajectory store [step][field][B] with fields (t, y[N], K[S][N]).
@@ -165,8 +184,12 @@ struct SharedRevArgs {
 };
 
 // Layout version of KernelSet: kernel tables made in a caller's translation unit
-// (VA_DEVICE_SYSTEM) are accepted only with the library's size and version.
-constexpr int32_t VA_KERNEL_TABLE_VERSION = 1;
+// (VA_DEVICE_SYSTEM) are accepted with the library's size and a version it knows.
+// Version 2 kernels read RevArgs::seeds_per_item and identity; version 1 kernels
+// (the same table and argument layout up to those members) sweep all seeds of an
+// instance one after the other and are never given either.
+constexpr int32_t VA_KERNEL_TABLE_VERSION = 2;
+constexpr int32_t VA_KERNEL_TABLE_OLDEST = 1;
 
 struct KernelSet {
     int32_t table_size = (int32_t)sizeof(KernelSet);
