@@ -231,6 +231,7 @@ __global__ void __launch_bounds__(256) k_order_hist(const int32_t *n_acc, const 
 // (the leading positions of the order that the long-instance kernel takes).
 constexpr int VA_LONG_BUCKET = 32;  // 256 attempts and more
 constexpr int VA_LONG_MAX = 256;    // one wave each
+constexpr int VA_REV_LONG = 4;      // where in va_handle::counters a reverse order's count lies
 
 __global__ void __launch_bounds__(VA_ORDER_BUCKETS)
 k_order_offsets(const int32_t *hist, int32_t *cursor, int32_t *n_long)
@@ -332,7 +333,7 @@ struct va_handle {
     int32_t *n_acc = nullptr, *n_rej = nullptr, *status = nullptr;
     // [0] fwd queue, [1] rev queue, [2] max steps, [3] active, [nlong_idx] long
     // instances at the head of order_fwd (from the previous forward's attempts),
-    // [11 - nlong_idx] those of order_fwd_next
+    // [11 - nlong_idx] those of order_fwd_next, [VA_REV_LONG] those of order
     int32_t *counters = nullptr;
     int32_t *order = nullptr;     // [B] reverse order, longest first
     int32_t *order_fwd = nullptr; // [B] next forward's order (previous attempts, longest first)
@@ -476,8 +477,8 @@ va_status order_by_length(va_handle *h, int mode, hipStream_t s)
     if (st) return st;
     const int gb = blocks_for(B, 256);
     int32_t *out = mode == 0 ? h->order : mode == 1 ? h->order_fwd : h->order_fwd_next;
-    int32_t *n_long = mode == 0 ? nullptr
-                      : h->counters + (mode == 1 ? h->nlong_idx : 11 - h->nlong_idx);
+    int32_t *n_long =
+        h->counters + (mode == 0 ? VA_REV_LONG : mode == 1 ? h->nlong_idx : 11 - h->nlong_idx);
     const int by = mode == 0 ? 0 : 1;
     if (mode != 0) h->ordered = true;
     hipLaunchKernelGGL(k_order_hist, dim3(gb), dim3(256), 0, s, h->n_acc, h->n_rej, h->status,
@@ -729,6 +730,12 @@ va_status reverse_persistent(va_handle *h, const double *p, int cost, const doub
         if ((st = params_instance_major(h, p, s))) return st;
         a.p = h->pim;
         if ((st = pbar_instance_major(h, a, nseed))) return st;
+    }
+    // one seed: the long instances at the head of the order take blocks of their own
+    if (nseed == 1 && h->ks.layout == 1 && h->pb.adaptive && va::rows_rev_head(h->ks.n) &&
+        h->block == 256) {
+        a.split = h->counters + VA_REV_LONG;
+        a.part = 2;
     }
     const int64_t lanes = std::min<int64_t>(h->lanes_rev, B * parts);
     VA_HIP(h->ks.rev(a, blocks_for(lanes, h->ks.slots(h->block)), h->block, s));

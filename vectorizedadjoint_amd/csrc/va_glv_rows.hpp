@@ -28,6 +28,7 @@
 // examples/GeneralizedLotkaVolterra/main.cpp:105-119 (system, parameter layout).
 #pragma once
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -170,12 +171,19 @@ __device__ __forceinline__ void bcast_group0(double x, double (&out)[NN])
     }
 }
 
-template <bool OneShot, int NN>
+// How a wave's lanes hold instances and exchange their vectors.
+enum class Lay {
+    Groups,  // 64/N groups of N consecutive lanes, vectors through an LDS slab
+    Rows,    // one group in each 16-lane row (N <= 16), vectors by DPP row broadcasts
+    One,     // group 0 alone (row broadcasts for N <= 16, else scalar registers)
+};
+
+template <Lay L, int NN>
 __device__ __forceinline__ void xchg(double *slab, int lane, int gbase, double x,
                                      double (&out)[NN])
 {
-    if constexpr (OneShot) bcast_group0<NN>(x, out);
-    else exchange<NN>(slab, lane, gbase, x, out);
+    if constexpr (L == Lay::Groups) exchange<NN>(slab, lane, gbase, x, out);
+    else bcast_group0<NN>(x, out);
 }
 
 // g_i = r_i + sum_j A_ij x_j in the reference functor's order
@@ -262,11 +270,20 @@ struct QueueRange {
     int64_t lo, hi;
 };
 
+// Part 2: positions below it are the first blocks', one each (half of the grid at
+// most), the queue holds the rest.
+__device__ __forceinline__ int head_blocks(const int32_t *split, int part)
+{
+    if (!split || part != 2) return 0;
+    const int half = (int)(gridDim.x / 2);
+    return *split < half ? *split : half;
+}
+
 __device__ __forceinline__ QueueRange queue_range(int64_t B, const int32_t *split, int part)
 {
     QueueRange q{0, B};
     if (split) {
-        const int64_t k = *split;
+        const int64_t k = part == 2 ? head_blocks(split, part) : *split;
         if (part == 0) q.hi = k < B ? k : B;
         else q.lo = k < B ? k : B;
     }
@@ -274,46 +291,82 @@ __device__ __forceinline__ QueueRange queue_range(int64_t B, const int32_t *spli
 }
 
 // ---------------------------------------------------------------------------
-// Forward sweep (persistent, refill per instance group)
+// Forward sweep (persistent, refill per instance group).
+//
+// What bounds it: the chain of attempts of the longest instances (a finite-time
+// blow-up takes some 1,500 attempts against a median of 72), each attempt some 400
+// dependent instructions.  In the Groups layout an exchange is an LDS round trip
+// of about 130 cycles for a wave with little else to do; in the Rows layout it is
+// one DPP move per component, with 4 instances per wave instead of 64/N, and with
+// the constants in vector registers.  So Rows serves forwards in index order
+// (no previous attempt counts: the long chains start anywhere in the queue),
+// Groups those with N > 16; One is the body of the long-instance kernels.
 // ---------------------------------------------------------------------------
-template <int NN, class Tab, bool Adaptive, bool OneShot>
+template <int NN, class Tab, bool Adaptive, Lay L>
 __device__ __forceinline__ void glv_rows_fwd_body(const FwdArgs &a, int64_t one)
 {
-    using L = GlvRows<NN>;
-    constexpr int F = L::F;
-    __shared__ double2 slab2[L::WAVES][32];
-    __shared__ double2 slabb2[L::WAVES][32];
-    __shared__ int gidx[L::WAVES][L::GPW];
+    constexpr int F = NN + 2, WAVES = 4;
+    constexpr bool kLds = L == Lay::Groups;
+    constexpr int G = L == Lay::Rows ? 16 : NN;      // lanes from group to group
+    constexpr int GPW = L == Lay::One ? 1 : 64 / G;  // groups per wave
+    __shared__ double2 slab2[kLds ? WAVES : 1][32];
+    __shared__ double2 slabb2[kLds ? WAVES : 1][32];
+    __shared__ int gidx[WAVES][64 / G];
 
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int grp = lane / NN, i = lane - grp * NN;
-    if (OneShot ? grp != 0 : grp >= L::GPW) return;
-    double *slab = reinterpret_cast<double *>(slab2[wv]);
-    double *slabb = reinterpret_cast<double *>(slabb2[wv]);
+    const int grp = lane / G, i = lane - grp * G;
+    if (grp >= GPW || i >= NN) return;
+    double *slab = reinterpret_cast<double *>(slab2[kLds ? wv : 0]);
+    double *slabb = reinterpret_cast<double *>(slabb2[kLds ? wv : 0]);
     const int gbase = grp * NN;
     const SolveParams sp = a.sp;
     const int64_t B = sp.B;
+    const int32_t cap = (int32_t)sp.cap;
     // For tableaus without FSAL the next step's f(y_{n+1}) is computed with the
     // error norm of the attempt (it does not depend on the step decision), so it
     // is off the accept path's critical chain; it is the same arithmetic as
     // evaluating it at the start of the next step.
     constexpr bool kSpec = Adaptive && !Tab::FSAL;
 
-    double Arow[NN], r = 0.0, y = 0.0, K[Tab::SF], ynew = 0.0, xerr = 0.0;
+    double Arow[NN], r = 0.0, y = 0.0, k0 = 0.0;  // k0 = f_i(y)
     double t = 0.0, dt = 0.0;
     int64_t b = 0;
     int32_t count = 0, rej = 0, tries = 0, st = LANE_OK;
-    bool new_step = true, have_k0 = false, need = true, taken = false;
-    double *rows = nullptr;
+    bool need = true, taken = false;
+    double *row = nullptr;  // row `count` of the instance
     double v[NN];
     const QueueRange q = queue_range(B, a.split, a.part);
-    const TabRegs<Tab, OneShot> tc;
+    const TabRegs<Tab, !kLds> tc;
+    const PowConsts<!kLds && Adaptive && Tab::SF <= 7> pc;
+
+    auto growth = [&](double x) {
+        xchg<L, NN>(slab, lane, gbase, x, v);
+        return growth_row<NN>(Arow, r, v);
+    };
+    // The head of the controlled loop at the point (t, y): false when the instance
+    // is done (or has no room for another step), else dt clipped to end at t1.
+    auto begin_step = [&]() {
+        const bool more = Adaptive ? less_with_sign(t, sp.t1, dt)
+                                   : less_eq_with_sign(t + sp.dt0, sp.t1, sp.dt0);
+        if (more && count >= cap) st = LANE_MAX_STEPS;
+        if constexpr (Adaptive)
+            if (less_with_sign(sp.t1, t + dt, dt)) dt = sp.t1 - t;
+        tries = 0;
+        return more && count < cap;
+    };
+    // (t, h) by every lane of the group, to the same address
+    auto store_row = [&](double h) {
+        row[0] = t;
+        row[1] = h;
+        row[2 + i] = y;
+    };
 
     for (;;) {
-        if constexpr (OneShot) __builtin_amdgcn_s_setprio(3);
+        bool finish = false;
+        if constexpr (L == Lay::One) __builtin_amdgcn_s_setprio(3);
         else if (!a.split) prioritise_long(!need && count + rej > VA_LONG_ATTEMPTS);
         if (need) {
-            if constexpr (OneShot) {
+            if constexpr (L == Lay::One) {
                 if (taken) break;
                 taken = true;
                 b = one;
@@ -325,116 +378,80 @@ __device__ __forceinline__ void glv_rows_fwd_body(const FwdArgs &a, int64_t one)
                 if (b >= q.hi) break;
                 if (a.order) b = a.order[b];
             }
-            r = growth_rate(param<NN, !OneShot>(a, i, b));
+            constexpr bool IM = L != Lay::One;
+            r = growth_rate(param<NN, IM>(a, i, b));
 #pragma unroll
-            for (int j = 0; j < NN; ++j) Arow[j] = param<NN, !OneShot>(a, NN * (i + 1) + j, b);
+            for (int j = 0; j < NN; ++j) Arow[j] = param<NN, IM>(a, NN * (i + 1) + j, b);
             y = a.y[(int64_t)i * B + b];
             t = sp.t0;
             dt = sp.dt0;
-            count = rej = tries = 0;
+            count = rej = 0;
             st = LANE_OK;
-            new_step = true;
-            have_k0 = false;
             need = false;
-            rows = a.traj + (size_t)b * (size_t)(sp.cap + 1) * F;
+            row = a.traj + (size_t)b * (size_t)(sp.cap + 1) * F;
             wait_vmem();
-        }
-        bool finish = false;
-        if (new_step) {
-            const bool more = Adaptive ? less_with_sign(t, sp.t1, dt)
-                                       : less_eq_with_sign(t + sp.dt0, sp.t1, sp.dt0);
-            if (!more) {
-                finish = true;
-            } else if (count >= sp.cap) {
-                st = LANE_MAX_STEPS;
-                finish = true;
-            } else {
-                double *row = rows + (size_t)count * F;
-                row[0] = t;
-                row[2 + i] = y;
-                if (Adaptive && less_with_sign(sp.t1, t + dt, dt)) dt = sp.t1 - t;
-                if ((!Tab::FSAL && !kSpec) || !have_k0) {
-                    xchg<OneShot, NN>(slab, lane, gbase, y, v);
-                    K[0] = y * growth_row<NN>(Arow, r, v);
-                    have_k0 = true;
-                }
-                tries = 0;
-                new_step = false;
-            }
+            k0 = y * growth(y);
+            finish = !begin_step();
         }
         if (!finish) {
             const double h = Adaptive ? dt : sp.dt0;
+            double K[Tab::SF];
+            K[0] = k0;
 #pragma unroll
             for (int m = 1; m < Tab::SF; ++m) {
                 double X = y;
 #pragma unroll
                 for (int j = 0; j < Tab::SF; ++j)
                     if (j < m && Tab::A[m][j] != 0.0) X = X + (tc.a[m][j] * h) * K[j];
-                xchg<OneShot, NN>(slab, lane, gbase, X, v);
-                K[m] = X * growth_row<NN>(Arow, r, v);
+                K[m] = X * growth(X);
             }
-            ynew = y;
+            double ynew = y;
 #pragma unroll
             for (int j = 0; j < Tab::S; ++j)
                 if (Tab::B[j] != 0.0) ynew = ynew + (tc.b[j] * h) * K[j];
+            bool accept = true, fail = false;
+            double k0n = 0.0;
             if constexpr (Adaptive) {
                 constexpr int j0 = ErrFirst<Tab>::value();
-                xerr = (tc.db[j0] * h) * K[j0];
+                double xerr = (tc.db[j0] * h) * K[j0];
 #pragma unroll
                 for (int j = j0 + 1; j < Tab::SF; ++j)
                     if (Tab::DB[j] != 0.0) xerr = xerr + (tc.db[j] * h) * K[j];
-                const double den = sp.atol + sp.rtol * (fabs(y) + h * fabs(K[0]));
-                double k0n = 0.0, ve[NN];
-                if constexpr (kSpec) {
-                    if constexpr (OneShot) {
-                        bcast_group0<NN>(ynew, v);
-                        bcast_group0<NN>(fabs(xerr) / den, ve);
-                    } else {
-                        exchange2<NN>(slab, slabb, lane, gbase, ynew, v, fabs(xerr) / den, ve);
-                    }
+                const double den = sp.atol + sp.rtol * (fabs(y) + h * fabs(k0));
+                double ve[NN];
+                if constexpr (kSpec && kLds) {
+                    exchange2<NN>(slab, slabb, lane, gbase, ynew, v, fabs(xerr) / den, ve);
                     k0n = ynew * growth_row<NN>(Arow, r, v);
                 } else {
-                    xchg<OneShot, NN>(slabb, lane, gbase, fabs(xerr) / den, ve);
+                    if constexpr (kSpec) k0n = ynew * growth(ynew);
+                    xchg<L, NN>(slabb, lane, gbase, fabs(xerr) / den, ve);
                 }
-                const double err = group_max<NN>(ve);
-                double dt_next;
-                if (!control_step<Tab>(dt, err, dt_next)) {
-                    ++rej;
-                } else {
-                    const double tn = t + dt;
-                    rows[(size_t)count * F + 1] = stored_step(tn, t);
-                    t = tn;
-                    y = ynew;
-                    if constexpr (Tab::FSAL) K[0] = K[Tab::SF - 1];
-                    if constexpr (kSpec) K[0] = k0n;
-                    ++count;
-                    new_step = true;
-                }
-                dt = dt_next;
-                ++tries;
-                if (tries > sp.max_attempts) {
-                    st = LANE_MAX_FAIL;
-                    finish = true;
-                }
-            } else {
-                const double tn = sp.t0 + (double)(count + 1) * sp.dt0;
-                rows[(size_t)count * F + 1] = stored_step(tn, t);
-                y = ynew;
-                if constexpr (Tab::FSAL) K[0] = K[Tab::SF - 1];
+                accept = control_step<Tab>(h, group_max<NN>(ve), dt, pc);
+                fail = ++tries > sp.max_attempts;
+            }
+            if (accept) {
                 ++count;
+                const double tn = Adaptive ? t + h : sp.t0 + (double)count * sp.dt0;
+                store_row(stored_step(tn, t));
+                row += F;
                 t = tn;
-                new_step = true;
+                y = ynew;
+                if constexpr (Tab::FSAL) k0 = K[Tab::SF - 1];
+                else if constexpr (kSpec) k0 = k0n;
+                else k0 = y * growth(y);
+                finish = !begin_step();
+            } else {
+                ++rej;
+            }
+            if (fail) {
+                st = LANE_MAX_FAIL;
+                finish = true;
             }
         }
         if (finish) {
             if (st == LANE_OK) {
-                double *row = rows + (size_t)count * F;
-                if (i == 0) {
-                    row[0] = t;
-                    row[1] = 0.0;
-                }
-                row[2 + i] = y;
-                xchg<OneShot, NN>(slab, lane, gbase, fabs(y), v);
+                store_row(0.0);
+                xchg<L, NN>(slab, lane, gbase, fabs(y), v);
                 bool fin = true;
 #pragma unroll
                 for (int j = 0; j < NN; ++j) fin = fin && (v[j] <= 1.7976931348623157e308);
@@ -452,11 +469,11 @@ __device__ __forceinline__ void glv_rows_fwd_body(const FwdArgs &a, int64_t one)
     }
 }
 
-template <int NN, class Tab, bool Adaptive>
+template <int NN, class Tab, bool Adaptive, Lay L>
 __global__ void __launch_bounds__(256) k_glv_rows_fwd(FwdArgs a)
 {
     if constexpr (Adaptive) load_ctrl_tables();
-    glv_rows_fwd_body<NN, Tab, Adaptive, false>(a, 0);
+    glv_rows_fwd_body<NN, Tab, Adaptive, L>(a, 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -518,19 +535,43 @@ __device__ __forceinline__ void glv_rows2_fwd_body(const FwdArgs &a)
     const int gbase = grp * NN;
     const SolveParams sp = a.sp;
     const int64_t B = sp.B;
+    const int32_t cap = (int32_t)sp.cap;
     constexpr bool kSpec = Adaptive && !Tab::FSAL;
 
-    double A[2][NN], r[2], y[2], K[SF][2], ynew[2], xerr[2];
+    double A[2][NN], r[2], y[2], k0[2];  // k0 = f(y)
     double t = 0.0, dt = 0.0;
     int64_t b = 0;
     int32_t count = 0, rej = 0, tries = 0, st = LANE_OK;
-    bool new_step = true, have_k0 = false, need = true;
-    double *rows = nullptr;
+    bool need = true;
+    double *row = nullptr;  // row `count` of the instance
     double v[NN];
     const QueueRange q = queue_range(B, a.split, a.part);
     const TabRegs<Tab, false> tc;
 
+    // f of the group's vector x into k
+    auto rhs = [&](const double (&x)[2], double (&k)[2]) {
+        exchange_pairs<NN>(slab, gbase, li, x[0], x[1], v);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) k[e] = x[e] * growth_row<NN>(A[e], r[e], v);
+    };
+    // as in glv_rows_fwd_body
+    auto begin_step = [&]() {
+        const bool more = Adaptive ? less_with_sign(t, sp.t1, dt)
+                                   : less_eq_with_sign(t + sp.dt0, sp.t1, sp.dt0);
+        if (more && count >= cap) st = LANE_MAX_STEPS;
+        if constexpr (Adaptive)
+            if (less_with_sign(sp.t1, t + dt, dt)) dt = sp.t1 - t;
+        tries = 0;
+        return more && count < cap;
+    };
+    auto store_row = [&](double h) {
+        row[0] = t;
+        row[1] = h;
+        *reinterpret_cast<double2 *>(row + 2 + i0) = make_double2(y[0], y[1]);
+    };
+
     for (;;) {
+        bool finish = false;
         if (!a.split) prioritise_long(!need && count + rej > VA_LONG_ATTEMPTS);
         if (need) {
             if (li == 0) gidx[wv][grp] = atomicAdd(a.counter, 1);
@@ -549,40 +590,17 @@ __device__ __forceinline__ void glv_rows2_fwd_body(const FwdArgs &a)
             }
             t = sp.t0;
             dt = sp.dt0;
-            count = rej = tries = 0;
+            count = rej = 0;
             st = LANE_OK;
-            new_step = true;
-            have_k0 = false;
             need = false;
-            rows = a.traj + (size_t)b * (size_t)(sp.cap + 1) * F;
+            row = a.traj + (size_t)b * (size_t)(sp.cap + 1) * F;
             wait_vmem();
-        }
-        bool finish = false;
-        if (new_step) {
-            const bool more = Adaptive ? less_with_sign(t, sp.t1, dt)
-                                       : less_eq_with_sign(t + sp.dt0, sp.t1, sp.dt0);
-            if (!more) {
-                finish = true;
-            } else if (count >= sp.cap) {
-                st = LANE_MAX_STEPS;
-                finish = true;
-            } else {
-                double *row = rows + (size_t)count * F;
-                row[0] = t;
-                *reinterpret_cast<double2 *>(row + 2 + i0) = make_double2(y[0], y[1]);
-                if (Adaptive && less_with_sign(sp.t1, t + dt, dt)) dt = sp.t1 - t;
-                if ((!Tab::FSAL && !kSpec) || !have_k0) {
-                    exchange_pairs<NN>(slab, gbase, li, y[0], y[1], v);
-#pragma unroll
-                    for (int e = 0; e < 2; ++e) K[0][e] = y[e] * growth_row<NN>(A[e], r[e], v);
-                    have_k0 = true;
-                }
-                tries = 0;
-                new_step = false;
-            }
+            rhs(y, k0);
+            finish = !begin_step();
         }
         if (!finish) {
             const double h = Adaptive ? dt : sp.dt0;
+            double K[SF][2] = {{k0[0], k0[1]}};
 #pragma unroll
             for (int m = 1; m < SF; ++m) {
                 double X[2] = {y[0], y[1]};
@@ -593,12 +611,9 @@ __device__ __forceinline__ void glv_rows2_fwd_body(const FwdArgs &a)
 #pragma unroll
                         for (int e = 0; e < 2; ++e) X[e] = X[e] + ah * K[j][e];
                     }
-                exchange_pairs<NN>(slab, gbase, li, X[0], X[1], v);
-#pragma unroll
-                for (int e = 0; e < 2; ++e) K[m][e] = X[e] * growth_row<NN>(A[e], r[e], v);
+                rhs(X, K[m]);
             }
-#pragma unroll
-            for (int e = 0; e < 2; ++e) ynew[e] = y[e];
+            double ynew[2] = {y[0], y[1]};
 #pragma unroll
             for (int j = 0; j < Tab::S; ++j)
                 if (Tab::B[j] != 0.0) {
@@ -606,9 +621,12 @@ __device__ __forceinline__ void glv_rows2_fwd_body(const FwdArgs &a)
 #pragma unroll
                     for (int e = 0; e < 2; ++e) ynew[e] = ynew[e] + bh * K[j][e];
                 }
+            bool accept = true, fail = false;
+            double k0n[2] = {0.0, 0.0};
             if constexpr (Adaptive) {
                 constexpr int j0 = ErrFirst<Tab>::value();
                 const double dh0 = tc.db[j0] * h;
+                double xerr[2], ratio[2], ve[NN];
 #pragma unroll
                 for (int e = 0; e < 2; ++e) xerr[e] = dh0 * K[j0][e];
 #pragma unroll
@@ -618,11 +636,9 @@ __device__ __forceinline__ void glv_rows2_fwd_body(const FwdArgs &a)
 #pragma unroll
                         for (int e = 0; e < 2; ++e) xerr[e] = xerr[e] + dh * K[j][e];
                     }
-                double ratio[2];
 #pragma unroll
                 for (int e = 0; e < 2; ++e)
-                    ratio[e] = fabs(xerr[e]) / (sp.atol + sp.rtol * (fabs(y[e]) + h * fabs(K[0][e])));
-                double k0n[2] = {0.0, 0.0}, ve[NN];
+                    ratio[e] = fabs(xerr[e]) / (sp.atol + sp.rtol * (fabs(y[e]) + h * fabs(k0[e])));
                 if constexpr (kSpec) {
                     exchange_pairs2<NN>(slab, slabb, gbase, li, ynew[0], ynew[1], v, ratio[0],
                                         ratio[1], ve);
@@ -631,50 +647,34 @@ __device__ __forceinline__ void glv_rows2_fwd_body(const FwdArgs &a)
                 } else {
                     exchange_pairs<NN>(slabb, gbase, li, ratio[0], ratio[1], ve);
                 }
-                const double err = group_max<NN>(ve);
-                double dt_next;
-                if (!control_step<Tab>(dt, err, dt_next)) {
-                    ++rej;
-                } else {
-                    const double tn = t + dt;
-                    rows[(size_t)count * F + 1] = stored_step(tn, t);
-                    t = tn;
-#pragma unroll
-                    for (int e = 0; e < 2; ++e) {
-                        y[e] = ynew[e];
-                        if constexpr (Tab::FSAL) K[0][e] = K[SF - 1][e];
-                        if constexpr (kSpec) K[0][e] = k0n[e];
-                    }
-                    ++count;
-                    new_step = true;
-                }
-                dt = dt_next;
-                ++tries;
-                if (tries > sp.max_attempts) {
-                    st = LANE_MAX_FAIL;
-                    finish = true;
-                }
-            } else {
-                const double tn = sp.t0 + (double)(count + 1) * sp.dt0;
-                rows[(size_t)count * F + 1] = stored_step(tn, t);
+                accept = control_step<Tab>(h, group_max<NN>(ve), dt);
+                fail = ++tries > sp.max_attempts;
+            }
+            if (accept) {
+                ++count;
+                const double tn = Adaptive ? t + h : sp.t0 + (double)count * sp.dt0;
+                store_row(stored_step(tn, t));
+                row += F;
+                t = tn;
 #pragma unroll
                 for (int e = 0; e < 2; ++e) {
                     y[e] = ynew[e];
-                    if constexpr (Tab::FSAL) K[0][e] = K[SF - 1][e];
+                    if constexpr (Tab::FSAL) k0[e] = K[SF - 1][e];
+                    if constexpr (kSpec) k0[e] = k0n[e];
                 }
-                ++count;
-                t = tn;
-                new_step = true;
+                if constexpr (!Tab::FSAL && !kSpec) rhs(y, k0);
+                finish = !begin_step();
+            } else {
+                ++rej;
+            }
+            if (fail) {
+                st = LANE_MAX_FAIL;
+                finish = true;
             }
         }
         if (finish) {
             if (st == LANE_OK) {
-                double *row = rows + (size_t)count * F;
-                if (li == 0) {
-                    row[0] = t;
-                    row[1] = 0.0;
-                }
-                *reinterpret_cast<double2 *>(row + 2 + i0) = make_double2(y[0], y[1]);
+                store_row(0.0);
                 exchange_pairs<NN>(slab, gbase, li, fabs(y[0]), fabs(y[1]), v);
                 bool fin = true;
 #pragma unroll
@@ -818,7 +818,7 @@ __device__ __forceinline__ void glv_rows_rev_body(const RevArgs &a, int64_t one,
             if (a.cost) {
                 const double yT = a.yT[(int64_t)i * B + b];
                 // terminal cost: J = fold over i in order, lambda_i from y_i(T)
-                xchg<OneShot, NN>(uslab, lane, gbase, yT, v);
+                xchg<OneShot ? Lay::One : Lay::Groups, NN>(uslab, lane, gbase, yT, v);
                 double J = 0.0;
 #pragma unroll
                 for (int j = 0; j < NN; ++j) {
@@ -929,12 +929,6 @@ __device__ __forceinline__ void glv_rows_rev_body(const RevArgs &a, int64_t one,
     }
 }
 
-template <int NN, class Tab>
-__global__ void __launch_bounds__(256) k_glv_rows_rev(RevArgs a)
-{
-    glv_rows_rev_body<NN, Tab, false>(a, 0, 0);
-}
-
 // ---------------------------------------------------------------------------
 // Instances expected to run long: queue positions [0, *split) of the forward
 // order, one block of three waves per instance.  Wave 0 runs the instance's
@@ -1002,7 +996,7 @@ __device__ __forceinline__ bool wait_above(Ring &R, int *ctr, int k)
 }
 
 // Wave 1: stage values of steps n_acc-1 .. 0 into the ring.
-template <int NN, class Tab>
+template <int NN, class Tab, bool IM>
 __device__ __forceinline__ void glv_long_stage(const RevArgs &a, int64_t b, StageRing<NN, Tab> &R)
 {
     constexpr int S = Tab::S, F = NN + 2;
@@ -1013,10 +1007,10 @@ __device__ __forceinline__ void glv_long_stage(const RevArgs &a, int64_t b, Stag
     const int64_t B = sp.B;
     const int32_t nacc = a.n_acc[b];
     if (a.status[b] != LANE_OK || nacc <= 0) return;
-    const double r = growth_rate(param<NN, false>(a, i, b));
+    const double r = growth_rate(param<NN, IM>(a, i, b));
     double Arow[NN], v[NN];
 #pragma unroll
-    for (int j = 0; j < NN; ++j) Arow[j] = param<NN, false>(a, NN * (i + 1) + j, b);
+    for (int j = 0; j < NN; ++j) Arow[j] = param<NN, IM>(a, NN * (i + 1) + j, b);
     const double *rows = a.traj + (size_t)b * (size_t)(sp.cap + 1) * F;
     const TabRegs<Tab, true> tc;
     // (h_n, y_n,i) of the next two steps, loaded ahead of use
@@ -1060,7 +1054,7 @@ __device__ __forceinline__ void glv_long_stage(const RevArgs &a, int64_t b, Stag
 // Wave 0 after the forward: terminal cost, then the adjoint recursion of steps
 // n_acc-1 .. 0 from the staged values (the backward of glv_rows_rev_body),
 // leaving each stage's products u in the step's slot for wave 2.
-template <int NN, class Tab>
+template <int NN, class Tab, bool IM>
 __device__ __forceinline__ void glv_long_backward(const RevArgs &a, int64_t b,
                                                   StageRing<NN, Tab> &R)
 {
@@ -1072,15 +1066,15 @@ __device__ __forceinline__ void glv_long_backward(const RevArgs &a, int64_t b,
     const double qnan = __builtin_nan("");
     if (a.status[b] != LANE_OK) {
         a.lambda[(int64_t)i * B + b] = qnan;
-        put_pbar_nan<NN, false>(a, 0, i, b);
-        for (int j = 0; j < NN; ++j) put_pbar_nan<NN, false>(a, 0, NN * (i + 1) + j, b);
+        put_pbar_nan<NN, IM>(a, 0, i, b);
+        for (int j = 0; j < NN; ++j) put_pbar_nan<NN, IM>(a, 0, NN * (i + 1) + j, b);
         if (a.cost) a.J[b] = qnan;
         return;
     }
     const TabRegs<Tab, true> tc;
     double Acol[NN], v[NN], vu[NN], lam;
 #pragma unroll
-    for (int j = 0; j < NN; ++j) Acol[j] = param<NN, false>(a, NN * (j + 1) + i, b);
+    for (int j = 0; j < NN; ++j) Acol[j] = param<NN, IM>(a, NN * (j + 1) + i, b);
     if (a.cost) {
         const double yT = a.yT[(int64_t)i * B + b];
         // terminal cost: J = fold over i in order, lambda_i from y_i(T)
@@ -1145,7 +1139,7 @@ __device__ __forceinline__ void glv_long_backward(const RevArgs &a, int64_t b,
 // Wave 2: dJ/dr_i and column i of dJ/dA from the products u of each step wave 0
 // has reversed, in wave 0's stage order (what glv_rows_rev_body accumulates
 // beside its recursion, the same operations in the same order).
-template <int NN, class Tab>
+template <int NN, class Tab, bool IM>
 __device__ __forceinline__ void glv_long_accumulate(const RevArgs &a, int64_t b,
                                                     StageRing<NN, Tab> &R)
 {
@@ -1184,9 +1178,38 @@ __device__ __forceinline__ void glv_long_accumulate(const RevArgs &a, int64_t b,
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         ring_store(&R.done, k + 1);
     }
-    put_pbar<NN, false>(a, 0, i, b, rbar);
+    put_pbar<NN, IM>(a, 0, i, b, rbar);
 #pragma unroll
-    for (int kk = 0; kk < NN; ++kk) put_pbar<NN, false>(a, 0, NN * (kk + 1) + i, b, Abar[kk]);
+    for (int kk = 0; kk < NN; ++kk) put_pbar<NN, IM>(a, 0, NN * (kk + 1) + i, b, Abar[kk]);
+}
+
+// The persistent reverse.  With part 2 (one seed) the head of the order, instances
+// of 256 and more accepted steps, is the first blocks': three of a block's waves
+// sweep one instance as in k_glv_rows_long, at the highest priority, and the block
+// then joins the others, which take the rest of the order from the start.  The
+// longest chain of a reverse without a long-instance kernel beside it so takes
+// 0.85 us per step instead of 1.6 (N=10, B=20000, index order: solve 3.7 -> 3.2 ms).
+template <int NN, class Tab, bool Head>
+__global__ void __launch_bounds__(256) k_glv_rows_rev(RevArgs a)
+{
+    if constexpr (Head) {
+        __shared__ StageRing<NN, Tab> ring;
+        if ((int)blockIdx.x < head_blocks(a.split, a.part)) {
+            const int64_t b = a.order[blockIdx.x];
+            if (threadIdx.x == 0) {
+                ring.avail = 0;
+                ring.uavail = 0;
+                ring.done = 0;
+                ring.abort = 0;
+            }
+            __syncthreads();
+            if (threadIdx.x < 64) glv_long_backward<NN, Tab, true>(a, b, ring);
+            else if (threadIdx.x < 128) glv_long_stage<NN, Tab, true>(a, b, ring);
+            else if (threadIdx.x < 192) glv_long_accumulate<NN, Tab, true>(a, b, ring);
+            __builtin_amdgcn_s_setprio(0);
+        }
+    }
+    glv_rows_rev_body<NN, Tab, false>(a, 0, 0);
 }
 
 template <int NN, class Tab>
@@ -1205,13 +1228,13 @@ __global__ void __launch_bounds__(192) k_glv_rows_long(FwdArgs fa, RevArgs ra)
         ring.done = 0;
         ring.abort = 0;
     }
-    if (threadIdx.x < 64) glv_rows_fwd_body<NN, Tab, true, true>(fa, b);
+    if (threadIdx.x < 64) glv_rows_fwd_body<NN, Tab, true, Lay::One>(fa, b);
     // the forward's rows, y(T), counts and status become visible to every wave
     // (the barrier orders the block's memory operations at workgroup scope)
     __syncthreads();
-    if (threadIdx.x < 64) glv_long_backward<NN, Tab>(ra, b, ring);
-    else if (threadIdx.x < 128) glv_long_stage<NN, Tab>(ra, b, ring);
-    else glv_long_accumulate<NN, Tab>(ra, b, ring);
+    if (threadIdx.x < 64) glv_long_backward<NN, Tab, false>(ra, b, ring);
+    else if (threadIdx.x < 128) glv_long_stage<NN, Tab, false>(ra, b, ring);
+    else glv_long_accumulate<NN, Tab, false>(ra, b, ring);
 }
 
 // The same instances in a forward alone (va_forward) and in a reverse alone
@@ -1225,7 +1248,7 @@ __global__ void __launch_bounds__(256) k_glv_rows_long_fwd(FwdArgs fa)
     load_ctrl_tables();
     const int64_t w = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     if (w >= *fa.split || w >= fa.sp.B) return;
-    glv_rows_fwd_body<NN, Tab, true, true>(fa, fa.order[w]);
+    glv_rows_fwd_body<NN, Tab, true, Lay::One>(fa, fa.order[w]);
 }
 
 // The reverse alone for one seed, as in k_glv_rows_long: one block of three
@@ -1247,9 +1270,9 @@ __global__ void __launch_bounds__(192) k_glv_rows_long_adj(RevArgs ra)
         ring.abort = 0;
     }
     __syncthreads();
-    if (threadIdx.x < 64) glv_long_backward<NN, Tab>(ra, b, ring);
-    else if (threadIdx.x < 128) glv_long_stage<NN, Tab>(ra, b, ring);
-    else glv_long_accumulate<NN, Tab>(ra, b, ring);
+    if (threadIdx.x < 64) glv_long_backward<NN, Tab, false>(ra, b, ring);
+    else if (threadIdx.x < 128) glv_long_stage<NN, Tab, false>(ra, b, ring);
+    else glv_long_accumulate<NN, Tab, false>(ra, b, ring);
 }
 
 template <int NN, class Tab>
@@ -1473,6 +1496,8 @@ __global__ void __launch_bounds__(256) k_glv_rows_plain_rev(PlainRevArgs a)
 
 template <int NN, class Tab, bool Ad, bool WithLong = true>
 struct LaunchGlvRows {
+    // three-wave blocks for the reverse's long head
+    static constexpr bool kHead = Ad && rows_rev_head(NN);
     // The persistent forward with two rows per lane where N is even and small
     // enough for both rows' parameters to stay in registers, when the instances
     // come longest-first (a.order): a wave then holds instances of similar
@@ -1480,6 +1505,12 @@ struct LaunchGlvRows {
     // longest of its instances, and 12 unordered instances per wave made the
     // first solve 18% slower than 6, so that forward keeps one row per lane.
     static constexpr bool kPairs = NN % 2 == 0 && NN <= 16;
+    // The Rows layout (N <= 16): waves that run two to a SIMD at most, four
+    // instances each.  It takes batches that are resident so, and index orders
+    // of any size where a wave of the Groups layout would hold no more than six
+    // instances.  (Forward of N=10, B=4096, chains of 1,500 attempts: 2.23 -> 1.81
+    // ms; B=20000 2.57 -> 2.13 ms; B=65536, a first solve, 4.2 -> 3.6 ms.)
+    static constexpr int kRowsWaves = 256 * 4 * 2;
     static hipError_t fwd(const FwdArgs &a, int grid, int block, hipStream_t s)
     {
         if constexpr (kPairs) {
@@ -1489,12 +1520,24 @@ struct LaunchGlvRows {
                 return hipGetLastError();
             }
         }
-        hipLaunchKernelGGL((k_glv_rows_fwd<NN, Tab, Ad>), dim3(grid), dim3(block), 0, s, a);
+        if constexpr (NN <= 16) {
+            if (a.sp.B <= 4 * kRowsWaves || (NN >= 10 && !a.order)) {
+                const int64_t instances = std::min<int64_t>((int64_t)grid * slots(block), a.sp.B);
+                const int64_t waves = std::min<int64_t>((instances + 3) / 4, kRowsWaves);
+                const int per_block = block / 64;
+                hipLaunchKernelGGL((k_glv_rows_fwd<NN, Tab, Ad, Lay::Rows>),
+                                   dim3((unsigned)((waves + per_block - 1) / per_block)),
+                                   dim3(block), 0, s, a);
+                return hipGetLastError();
+            }
+        }
+        hipLaunchKernelGGL((k_glv_rows_fwd<NN, Tab, Ad, Lay::Groups>), dim3(grid), dim3(block), 0,
+                           s, a);
         return hipGetLastError();
     }
     static hipError_t rev(const RevArgs &a, int grid, int block, hipStream_t s)
     {
-        hipLaunchKernelGGL((k_glv_rows_rev<NN, Tab>), dim3(grid), dim3(block), 0, s, a);
+        hipLaunchKernelGGL((k_glv_rows_rev<NN, Tab, kHead>), dim3(grid), dim3(block), 0, s, a);
         return hipGetLastError();
     }
     static hipError_t lng(const FwdArgs &fa, const RevArgs &ra, int grid, int block,
@@ -1537,14 +1580,14 @@ struct LaunchGlvRows {
             e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_glv_rows2_fwd<NN, Tab, Ad>,
                                                              block, 0);
         else
-            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_glv_rows_fwd<NN, Tab, Ad>,
-                                                             block, 0);
+            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &nb, k_glv_rows_fwd<NN, Tab, Ad, Lay::Groups>, block, 0);
         return e == hipSuccess ? nb : 1;
     }
     static int occ_rev(int block)
     {
         int nb = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_glv_rows_rev<NN, Tab>, block, 0) !=
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_glv_rows_rev<NN, Tab, kHead>, block, 0) !=
             hipSuccess)
             return 1;
         return nb;

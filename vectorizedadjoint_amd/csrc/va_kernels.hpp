@@ -50,8 +50,8 @@ struct RevArgs {
     int32_t nout;
     int32_t *counter;
     const int32_t *order;  // [B] or null: the k-th instance taken is order[k]
-    const int32_t *split = nullptr;  // as in FwdArgs
-    int32_t part = 0;
+    const int32_t *split = nullptr;  // as in FwdArgs; part 2 (rows_rev_head): the first blocks
+    int32_t part = 0;                // take [0, *split) of the order, the queue holds the rest
     int32_t *pbar_set = nullptr;     // [B] or null
     // (cost == 0) seeds that one work item takes: 0 all of them, else items are
     // (instance, group of so many seeds) pairs.  See seeds_per_item() in va_capi.cpp.
@@ -73,6 +73,10 @@ __host__ __device__ inline RevItems rev_items(const RevArgs &a)
     r.parts = (r.seeds + r.per - 1) / r.per;
     return r;
 }
+
+// Whether the adaptive Lotka-Volterra row kernels of N species take part 2 in their
+// reverse (the long instances' waves exchange by row broadcasts: N <= 16).
+constexpr bool rows_rev_head(int n) { return n <= 16; }
 
 // Plain form: one launch per accepted step, state in HBM, no refill, full
 // trajectory store [step][field][B] with fields (t, y[N], K[S][N]).
