@@ -60,22 +60,48 @@ __global__ void k_copy_f64(double *dst, const double *src, int64_t n)
     if (i < n) dst[i] = src[i];
 }
 
+// A call's start: the work counters cleared, with the order kernels' histograms
+// behind them (the counts of long instances between the two stay), and y(T) := y0
+// where they differ (nd doubles, else 0).
+constexpr int VA_COUNTERS = 8;         // va_handle::counters
+constexpr int VA_ORDER_BUCKETS = 256;  // = the block size of the order kernels
+constexpr int VA_ORDER_INTS = 4 * VA_ORDER_BUCKETS;  // two orders' histograms and cursors
+constexpr int VA_WORK_INTS = VA_COUNTERS + VA_ORDER_INTS;
+
+__device__ __forceinline__ void clear_work(int32_t *counters)
+{
+    for (int k = threadIdx.x; k < VA_WORK_INTS; k += blockDim.x)
+        if (k < 4 || k >= VA_COUNTERS) counters[k] = 0;
+}
+
+__global__ void k_prologue(int32_t *counters, double *yT, const double *y0, int64_t nd)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < nd) yT[i] = y0[i];
+    if (blockIdx.x == 0) clear_work(counters);
+}
+
 __global__ void k_iota_i32(int32_t *p, int64_t n)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = (int32_t)i;
 }
 
-// The per-instance counts and status to the caller's arrays (any may be null).
-__global__ void k_copy_counts(int32_t *n_acc, int32_t *n_rej, int32_t *status,
-                              const int32_t *s_acc, const int32_t *s_rej, const int32_t *s_st,
-                              int64_t n)
+// The per-instance counts and status, and the caller's arrays for them (any may
+// be null).
+struct CountsOut {
+    int32_t *n_acc = nullptr, *n_rej = nullptr, *status = nullptr;
+    bool any() const { return n_acc || n_rej || status; }
+};
+
+__global__ void k_copy_counts(CountsOut out, const int32_t *s_acc, const int32_t *s_rej,
+                              const int32_t *s_st, int64_t n)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    if (n_acc) n_acc[i] = s_acc[i];
-    if (n_rej) n_rej[i] = s_rej[i];
-    if (status) status[i] = s_st[i];
+    if (out.n_acc) out.n_acc[i] = s_acc[i];
+    if (out.n_rej) out.n_rej[i] = s_rej[i];
+    if (out.status) out.status[i] = s_st[i];
 }
 
 __global__ void k_identity_seeds(double *lambda, int n, int64_t B)
@@ -141,8 +167,8 @@ __global__ void __launch_bounds__(256) k_to_instance_major(const double *src, do
 }
 
 // A split solve's prologue in one launch: the parameter copy above, y(T) := y0
-// (when they differ) and cleared marks for the block's instances, and, in block
-// 0, the cleared work counters [0, 4).
+// (when they differ) and cleared marks (when given) for the block's instances,
+// and, in block 0, the cleared work counters and histograms.
 __global__ void __launch_bounds__(256) k_split_prologue(const double *p, double *pim, int64_t P,
                                                         int64_t B, const double *y0, double *yT,
                                                         int n, int32_t *marks, int32_t *counters)
@@ -154,8 +180,8 @@ __global__ void __launch_bounds__(256) k_split_prologue(const double *p, double 
     const int bb = threadIdx.x & 31;
     if (y0 != yT && bb < nb)
         for (int i = threadIdx.x >> 5; i < n; i += 8) yT[(int64_t)i * B + b0 + bb] = y0[(int64_t)i * B + b0 + bb];
-    if ((int)threadIdx.x < nb) marks[b0 + threadIdx.x] = 0;
-    if (blockIdx.x == 0 && threadIdx.x < 4) counters[threadIdx.x] = 0;
+    if (marks && (int)threadIdx.x < nb) marks[b0 + threadIdx.x] = 0;
+    if (blockIdx.x == 0) clear_work(counters);
 }
 
 // dJ/dp sums of the row kernels, instance-major [nout][B][P], into mu
@@ -200,7 +226,17 @@ __global__ void __launch_bounds__(256) k_from_instance_major(const double *src, 
 // order is arbitrary.  Reverse order (mode 0): accepted steps, failed instances
 // last (they only write NaN).  Forward order (mode 1): attempts, every status.
 // Each instance's result does not depend on the order.
-constexpr int VA_ORDER_BUCKETS = 256;  // = the block size of the order kernels
+//
+// Two launches build one order or both (modes: a bit mask): the histograms, with
+// the caller's counts copied beside them, and the scatter, whose blocks each form
+// the buckets' offsets for themselves (five launches and the copy took 25 us at
+// the end of a solve, nine and the copy where the reverse had an order of its
+// own).  A thread takes up to VA_ORDER_ITEMS instances of a large batch: fewer
+// atomics on a bucket's counter, and an order that keeps runs of neighbouring
+// instances, whose rows are neighbours in memory.  With one instance per thread
+// the lanes of a wave had rows all over a 50 GB store (oscillator, B=2^20: solve
+// 33.8 ms so, 26.7 ms with 16, most of it address translation).
+constexpr int VA_ORDER_ITEMS = 16;
 
 __device__ __forceinline__ int order_bucket(const int32_t *n_acc, const int32_t *n_rej,
                                             const int32_t *status, int64_t b, int mode)
@@ -212,65 +248,85 @@ __device__ __forceinline__ int order_bucket(const int32_t *n_acc, const int32_t 
     return k < VA_ORDER_BUCKETS - 1 ? k : VA_ORDER_BUCKETS - 1;
 }
 
-__global__ void __launch_bounds__(256) k_order_hist(const int32_t *n_acc, const int32_t *n_rej,
-                                                    const int32_t *status, int64_t B, int mode,
-                                                    int32_t *hist)
+struct OrderArgs {
+    const int32_t *n_acc, *n_rej, *status;
+    int64_t B;
+    int modes;       // bit 0: the reverse order, bit 1: the forward order
+    int items;       // instances per thread, at most VA_ORDER_ITEMS
+    int32_t *work;   // per mode a histogram and cursors, cleared before
+    int32_t *order[2], *n_long[2];
+};
+
+__global__ void __launch_bounds__(VA_ORDER_BUCKETS) k_order_hist(OrderArgs a, CountsOut out)
 {
-    __shared__ int32_t cnt[VA_ORDER_BUCKETS];
-    if (threadIdx.x < VA_ORDER_BUCKETS) cnt[threadIdx.x] = 0;
+    __shared__ int32_t cnt[2][VA_ORDER_BUCKETS];
+    cnt[0][threadIdx.x] = cnt[1][threadIdx.x] = 0;
     __syncthreads();
-    const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < B) atomicAdd(&cnt[order_bucket(n_acc, n_rej, status, b, mode)], 1);
+    const int64_t b0 = (int64_t)blockIdx.x * VA_ORDER_BUCKETS * a.items + threadIdx.x;
+    for (int j = 0; j < a.items; ++j) {
+        const int64_t b = b0 + (int64_t)j * VA_ORDER_BUCKETS;
+        if (b >= a.B) break;
+        for (int m = 0; m < 2; ++m)
+            if (a.modes >> m & 1)
+                atomicAdd(&cnt[m][order_bucket(a.n_acc, a.n_rej, a.status, b, m)], 1);
+        if (out.n_acc) out.n_acc[b] = a.n_acc[b];
+        if (out.n_rej) out.n_rej[b] = a.n_rej[b];
+        if (out.status) out.status[b] = a.status[b];
+    }
     __syncthreads();
-    if (threadIdx.x < VA_ORDER_BUCKETS && cnt[threadIdx.x])
-        atomicAdd(&hist[threadIdx.x], cnt[threadIdx.x]);
+    for (int m = 0; m < 2; ++m)
+        if (cnt[m][threadIdx.x])
+            atomicAdd(&a.work[2 * m * VA_ORDER_BUCKETS + threadIdx.x], cnt[m][threadIdx.x]);
 }
 
-// cursor[k] = number of instances in buckets above k (longest bucket first).
-// With n_long: the instances in buckets >= VA_LONG_BUCKET, at most VA_LONG_MAX
-// (the leading positions of the order that the long-instance kernel takes).
-constexpr int VA_LONG_BUCKET = 32;  // 256 attempts and more
-constexpr int VA_LONG_MAX = 256;    // one wave each
+// The instances in buckets >= VA_LONG_BUCKET, at most VA_LONG_MAX, are the head of
+// an order that the long-instance kernels take; their count goes to n_long.
+constexpr int VA_LONG_BUCKET = 32;  // 256 attempts (or accepted steps) and more
+constexpr int VA_LONG_MAX = 256;    // one block each
 constexpr int VA_REV_LONG = 4;      // where in va_handle::counters a reverse order's count lies
 
-__global__ void __launch_bounds__(VA_ORDER_BUCKETS)
-k_order_offsets(const int32_t *hist, int32_t *cursor, int32_t *n_long)
+__global__ void __launch_bounds__(VA_ORDER_BUCKETS) k_order_scatter(OrderArgs a)
 {
-    // one thread per bucket: suffix sums by doubling steps
-    __shared__ int32_t sfx[VA_ORDER_BUCKETS];
+    __shared__ int32_t sfx[VA_ORDER_BUCKETS], cnt[VA_ORDER_BUCKETS];
     const int k = threadIdx.x;
-    const int32_t own = hist[k];
-    sfx[k] = own;
-    __syncthreads();
-    for (int d = 1; d < VA_ORDER_BUCKETS; d *= 2) {
-        const int32_t v = k + d < VA_ORDER_BUCKETS ? sfx[k + d] : 0;
+    const int64_t b0 = (int64_t)blockIdx.x * VA_ORDER_BUCKETS * a.items + k;
+    for (int m = 0; m < 2; ++m) {
+        if (!(a.modes >> m & 1)) continue;
+        int32_t *hist = a.work + 2 * m * VA_ORDER_BUCKETS, *cursor = hist + VA_ORDER_BUCKETS;
+        // instances in buckets above k (longest bucket first): suffix sums by
+        // doubling steps
+        const int32_t own = hist[k];
+        sfx[k] = own;
+        cnt[k] = 0;
         __syncthreads();
-        sfx[k] += v;
+        for (int d = 1; d < VA_ORDER_BUCKETS; d *= 2) {
+            const int32_t v = k + d < VA_ORDER_BUCKETS ? sfx[k + d] : 0;
+            __syncthreads();
+            sfx[k] += v;
+            __syncthreads();
+        }
+        if (blockIdx.x == 0 && k == VA_LONG_BUCKET)
+            *a.n_long[m] = sfx[k] < VA_LONG_MAX ? sfx[k] : VA_LONG_MAX;
+        int bucket[VA_ORDER_ITEMS], rank[VA_ORDER_ITEMS];
+#pragma unroll
+        for (int j = 0; j < VA_ORDER_ITEMS; ++j) {
+            const int64_t b = b0 + (int64_t)j * VA_ORDER_BUCKETS;
+            if (j < a.items && b < a.B) {
+                bucket[j] = order_bucket(a.n_acc, a.n_rej, a.status, b, m);
+                rank[j] = atomicAdd(&cnt[bucket[j]], 1);
+            }
+        }
+        __syncthreads();
+        // the block's share of each bucket: first place of its instances
+        sfx[k] += (cnt[k] ? atomicAdd(&cursor[k], cnt[k]) : 0) - own;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < VA_ORDER_ITEMS; ++j) {
+            const int64_t b = b0 + (int64_t)j * VA_ORDER_BUCKETS;
+            if (j < a.items && b < a.B) a.order[m][sfx[bucket[j]] + rank[j]] = (int32_t)b;
+        }
         __syncthreads();
     }
-    cursor[k] = sfx[k] - own;
-    if (k == VA_LONG_BUCKET && n_long) *n_long = sfx[k] < VA_LONG_MAX ? sfx[k] : VA_LONG_MAX;
-}
-
-__global__ void __launch_bounds__(256) k_order_scatter(const int32_t *n_acc,
-                                                       const int32_t *n_rej,
-                                                       const int32_t *status, int64_t B,
-                                                       int mode, int32_t *cursor, int32_t *order)
-{
-    __shared__ int32_t cnt[VA_ORDER_BUCKETS], base[VA_ORDER_BUCKETS];
-    if (threadIdx.x < VA_ORDER_BUCKETS) cnt[threadIdx.x] = 0;
-    __syncthreads();
-    const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int k = 0, r = 0;
-    if (b < B) {
-        k = order_bucket(n_acc, n_rej, status, b, mode);
-        r = atomicAdd(&cnt[k], 1);
-    }
-    __syncthreads();
-    if (threadIdx.x < VA_ORDER_BUCKETS && cnt[threadIdx.x])
-        base[threadIdx.x] = atomicAdd(&cursor[threadIdx.x], cnt[threadIdx.x]);
-    __syncthreads();
-    if (b < B) order[base[k] + r] = (int32_t)b;
 }
 
 // Digest of each instance's stored step sequence: d = 0x9E3779B97F4A7C15, then for
@@ -333,7 +389,8 @@ struct va_handle {
     int32_t *n_acc = nullptr, *n_rej = nullptr, *status = nullptr;
     // [0] fwd queue, [1] rev queue, [2] max steps, [3] active, [nlong_idx] long
     // instances at the head of order_fwd (from the previous forward's attempts),
-    // [11 - nlong_idx] those of order_fwd_next, [VA_REV_LONG] those of order
+    // [11 - nlong_idx] those of order_fwd_next, [VA_REV_LONG] those of order; then
+    // the order kernels' histograms and cursors
     int32_t *counters = nullptr;
     int32_t *order = nullptr;     // [B] reverse order, longest first
     int32_t *order_fwd = nullptr; // [B] next forward's order (previous attempts, longest first)
@@ -341,7 +398,6 @@ struct va_handle {
     // reverse still reads order_fwd; the two are swapped when it returns
     int32_t *order_fwd_next = nullptr;
     int nlong_idx = 5;
-    int32_t *order_tmp = nullptr; // [2 * VA_ORDER_BUCKETS] histogram, cursors
     // observed solves
     int64_t lanes_obs_fwd = 0, lanes_obs_rev = 0;
     int32_t obs_ckpt = 0, obs_slots = 0, obs_stride_max = 0;
@@ -446,7 +502,6 @@ void release(va_handle *h)
     hipFree(h->order);
     hipFree(h->order_fwd);
     hipFree(h->order_fwd_next);
-    hipFree(h->order_tmp);
     hipFree(h->obs_ck);
     hipFree(h->obs_seg);
     hipFree(h->obs_ck2);
@@ -466,32 +521,41 @@ void release(va_handle *h)
     if (h->host_counter) hipHostFree(h->host_counter);
 }
 
-// Longest-first order over the instances of the last forward: mode 0 into
-// h->order (the reverse, by accepted steps), mode 1 into h->order_fwd (the next
-// forward, by attempts, with its count of long instances), mode 2 as mode 1 into
-// h->order_fwd_next.
-va_status order_by_length(va_handle *h, int mode, hipStream_t s)
+va_status clear_and_copy(va_handle *h, double *yT, const double *y0, hipStream_t s)
 {
-    const int64_t B = h->pb.batch;
-    va_status st = fill_i32(h->order_tmp, 0, 2 * VA_ORDER_BUCKETS, s);
-    if (st) return st;
-    const int gb = blocks_for(B, 256);
-    int32_t *out = mode == 0 ? h->order : mode == 1 ? h->order_fwd : h->order_fwd_next;
-    int32_t *n_long =
-        h->counters + (mode == 0 ? VA_REV_LONG : mode == 1 ? h->nlong_idx : 11 - h->nlong_idx);
-    const int by = mode == 0 ? 0 : 1;
-    if (mode != 0) h->ordered = true;
-    hipLaunchKernelGGL(k_order_hist, dim3(gb), dim3(256), 0, s, h->n_acc, h->n_rej, h->status,
-                       B, by, h->order_tmp);
-    hipLaunchKernelGGL(k_order_offsets, dim3(1), dim3(VA_ORDER_BUCKETS), 0, s, h->order_tmp,
-                       h->order_tmp + VA_ORDER_BUCKETS, n_long);
-    hipLaunchKernelGGL(k_order_scatter, dim3(gb), dim3(256), 0, s, h->n_acc, h->n_rej,
-                       h->status, B, by, h->order_tmp + VA_ORDER_BUCKETS, out);
+    const int64_t nd = yT != y0 ? (int64_t)h->ks.n * h->pb.batch : 0;
+    hipLaunchKernelGGL(k_prologue, dim3(std::max(1, blocks_for(nd, 256))), dim3(256), 0, s,
+                       h->counters, yT, y0, nd);
     VA_HIP(hipGetLastError());
     return VA_OK;
 }
 
-va_status order_longest_first(va_handle *h, hipStream_t s) { return order_by_length(h, 0, s); }
+// Longest-first orders over the instances of the forward that just ran, once per
+// forward (its prologue cleared the histograms), with the caller's counts copied:
+// bit 0 of modes into h->order (the reverse, by accepted steps), bit 1 into
+// h->order_fwd (the next forward, by attempts) or, with next, into
+// h->order_fwd_next, each with its count of long instances.
+va_status build_orders(va_handle *h, int modes, bool next, const CountsOut &out, hipStream_t s)
+{
+    OrderArgs a;
+    a.n_acc = h->n_acc;
+    a.n_rej = h->n_rej;
+    a.status = h->status;
+    a.B = h->pb.batch;
+    a.modes = modes;
+    a.items = (int)std::min<int64_t>(VA_ORDER_ITEMS, std::max<int64_t>(1, a.B >> 14));
+    a.work = h->counters + VA_COUNTERS;
+    a.order[0] = h->order;
+    a.n_long[0] = h->counters + VA_REV_LONG;
+    a.order[1] = next ? h->order_fwd_next : h->order_fwd;
+    a.n_long[1] = h->counters + (next ? 11 - h->nlong_idx : h->nlong_idx);
+    if (modes & 2) h->ordered = true;
+    const int grid = blocks_for(a.B, VA_ORDER_BUCKETS * a.items);
+    hipLaunchKernelGGL(k_order_hist, dim3(grid), dim3(VA_ORDER_BUCKETS), 0, s, a, out);
+    hipLaunchKernelGGL(k_order_scatter, dim3(grid), dim3(VA_ORDER_BUCKETS), 0, s, a);
+    VA_HIP(hipGetLastError());
+    return VA_OK;
+}
 
 // Forwards take instances longest-first by an earlier forward's attempts unless
 // the caller asked for index order: where instances are refilled (more
@@ -522,6 +586,13 @@ bool reuse_order(const va_handle *h, int64_t lanes)
 bool split_solve(const va_handle *h)
 {
     return h->side && reuse_order(h, h->lanes_fwd);
+}
+
+// A reverse beside a long-instance kernel takes the order that its forward left
+// for the next one; any other has h->order.
+bool split_reverse(const va_handle *h)
+{
+    return h->side && h->ks.long_rev && order_wanted(h, h->lanes_fwd);
 }
 
 // Blocks of a persistent kernel beside a long-instance kernel: all of its
@@ -624,11 +695,24 @@ va_status bulk_instance_major(va_handle *h, const double *p, va::RevArgs *r, int
     return VA_OK;
 }
 
-va_status forward_persistent(va_handle *h, double *y, const double *p, hipStream_t s)
+// y := y0 (the same array for a caller that has it in place), then the sweep, the
+// orders it leaves and the caller's counts.
+va_status forward_persistent(va_handle *h, double *y, const double *y0, const double *p,
+                             const CountsOut &out, hipStream_t s)
 {
     const int64_t B = h->pb.batch;
-    va_status st = fill_i32(h->counters, 0, 4, s);
-    if (st) return st;
+    va_status st = VA_OK;
+    const bool split = split_solve(h) && h->ks.long_fwd;
+    const bool im = instance_major(h);
+    if (im && !split) {
+        // in one launch: parameters instance-major, y := y0, cleared counters
+        hipLaunchKernelGGL(k_split_prologue, dim3(blocks_for(B, VA_TILE_B)), dim3(256), 0, s, p,
+                           h->pim, (int64_t)h->ks.np, B, y0, y, h->ks.n, (int32_t *)nullptr,
+                           h->counters);
+        VA_HIP(hipGetLastError());
+    } else if ((st = clear_and_copy(h, y, y0, s))) {
+        return st;
+    }
     va::FwdArgs a;
     a.sp = solve_params(h);
     a.y = y;
@@ -639,11 +723,10 @@ va_status forward_persistent(va_handle *h, double *y, const double *p, hipStream
     a.status = h->status;
     a.counter = h->counters + 0;
     a.max_steps_seen = h->counters + 2;
-    const bool im = instance_major(h);
     const bool reuse = reuse_order(h, h->lanes_fwd);
     a.order = reuse ? h->order_fwd : nullptr;
     const int64_t lanes = std::min<int64_t>(h->lanes_fwd, B);
-    if (split_solve(h) && h->ks.long_fwd) {
+    if (split) {
         a.split = h->counters + h->nlong_idx;
         a.part = 1;
         if ((st = fork_side(h, s))) return st;
@@ -656,14 +739,11 @@ va_status forward_persistent(va_handle *h, double *y, const double *p, hipStream
         VA_HIP(h->ks.fwd(ab, bulk_grid(h, h->lanes_fwd), h->block, h->side));
         if ((st = join_side(h, s))) return st;
     } else {
-        if (im) {
-            if ((st = params_instance_major(h, p, s))) return st;
-            a.p = h->pim;
-        }
+        if (im) a.p = h->pim;
         VA_HIP(h->ks.fwd(a, blocks_for(lanes, h->ks.slots(h->block)), h->block, s));
     }
-    if (order_wanted(h, h->lanes_fwd)) return order_by_length(h, 1, s);
-    return VA_OK;
+    const int modes = (order_wanted(h, h->lanes_fwd) ? 2 : 0) | (split_reverse(h) ? 0 : 1);
+    return build_orders(h, modes, false, out, s);
 }
 
 // Seeds a work item of a reverse of nout seeds takes.  The Lotka-Volterra groups
@@ -681,17 +761,18 @@ int32_t seeds_per_item(const va_handle *h, int nout)
 }
 
 // identity: the seeds are the unit vectors (lambda is not used, mu = 0.0 + sum).
+// same_call: the forward of this call precedes it on s (its counters are clear and
+// h->pim holds p).
 va_status reverse_persistent(va_handle *h, const double *p, int cost, const double *cost_w,
                              const double *yT, double *J, double *lambda, double *mu, int nout,
-                             hipStream_t s, bool identity = false)
+                             hipStream_t s, bool identity = false, bool same_call = false)
 {
     const int64_t B = h->pb.batch;
-    va_status st = fill_i32(h->counters + 1, 0, 1, s);
-    if (st) return st;
+    va_status st = VA_OK;
+    if (!same_call && (st = fill_i32(h->counters + 1, 0, 1, s))) return st;
     // With the split schedule the last forward left its own instances
     // longest-first by attempts in order_fwd, and their long head counted.
-    const bool split = split_solve(h) && h->ks.long_rev;
-    if (!split && (st = order_longest_first(h, s))) return st;
+    const bool split = split_reverse(h);
     va::RevArgs a;
     a.sp = solve_params(h);
     a.order = split ? h->order_fwd : h->order;
@@ -727,7 +808,7 @@ va_status reverse_persistent(va_handle *h, const double *p, int cost, const doub
         return join_side(h, s);
     }
     if (im) {
-        if ((st = params_instance_major(h, p, s))) return st;
+        if (!same_call && (st = params_instance_major(h, p, s))) return st;
         a.p = h->pim;
         if ((st = pbar_instance_major(h, a, nseed))) return st;
     }
@@ -743,25 +824,14 @@ va_status reverse_persistent(va_handle *h, const double *p, int cost, const doub
     return VA_OK;
 }
 
-va_status copy_out(va_handle *h, int32_t *n_acc, int32_t *n_rej, int32_t *lane_status,
-                   hipStream_t s);
-
 va_status solve_split(va_handle *h, const double *y0, double *yT, const double *p, int cost,
                       const double *cost_w, double *J, double *dJdy0, double *dJdp,
-                      int32_t *n_accepted, int32_t *n_rejected, int32_t *lane_status,
-                      hipStream_t s)
+                      const CountsOut &out, hipStream_t s)
 {
     va_status st = VA_OK;
     const int64_t B = h->pb.batch;
     const bool im = instance_major(h);
-    if (!im) {
-        if ((st = fill_i32(h->counters, 0, 4, s))) return st;
-        if (yT != y0) {
-            hipLaunchKernelGGL(k_copy_f64, dim3(blocks_for((int64_t)h->ks.n * B, 256)), dim3(256),
-                               0, s, yT, y0, (int64_t)h->ks.n * B);
-            VA_HIP(hipGetLastError());
-        }
-    }
+    if (!im && (st = clear_and_copy(h, yT, y0, s))) return st;
     va::FwdArgs fa;
     fa.sp = solve_params(h);
     fa.y = yT;
@@ -821,16 +891,12 @@ va_status solve_split(va_handle *h, const double *y0, double *yT, const double *
     if (ahead) {
         VA_HIP(hipEventRecord(h->ev_fwd, h->side));
         VA_HIP(hipStreamWaitEvent(s, h->ev_fwd, 0));
-        if ((st = order_by_length(h, 2, s))) return st;
-        if ((st = copy_out(h, n_accepted, n_rejected, lane_status, s))) return st;
+        if ((st = build_orders(h, 2, true, out, s))) return st;
     }
     VA_HIP(h->ks.rev(rb, bulk_grid(h, h->lanes_rev), h->block, h->side));
     if (im && (st = pbar_to_mu(h, dJdp, 1, cost == 0, h->side, h->pbar_set))) return st;
     if ((st = join_side(h, s))) return st;
-    if (!ahead) {
-        if ((st = order_by_length(h, 1, s))) return st;
-        return copy_out(h, n_accepted, n_rejected, lane_status, s);
-    }
+    if (!ahead) return build_orders(h, 2, false, out, s);
     std::swap(h->order_fwd, h->order_fwd_next);
     h->nlong_idx = 11 - h->nlong_idx;
     return VA_OK;
@@ -916,13 +982,12 @@ va_status reverse_plain_seed(va_handle *h, const double *p, double *lambda, doub
     return VA_OK;
 }
 
-va_status copy_out(va_handle *h, int32_t *n_acc, int32_t *n_rej, int32_t *lane_status,
-                   hipStream_t s)
+va_status copy_out(va_handle *h, const CountsOut &out, hipStream_t s)
 {
     const int64_t B = h->pb.batch;
-    if (!n_acc && !n_rej && !lane_status) return VA_OK;
-    hipLaunchKernelGGL(k_copy_counts, dim3(blocks_for(B, 256)), dim3(256), 0, s, n_acc, n_rej,
-                       lane_status, h->n_acc, h->n_rej, h->status, B);
+    if (!out.any()) return VA_OK;
+    hipLaunchKernelGGL(k_copy_counts, dim3(blocks_for(B, 256)), dim3(256), 0, s, out, h->n_acc,
+                       h->n_rej, h->status, B);
     VA_HIP(hipGetLastError());
     return VA_OK;
 }
@@ -1199,11 +1264,10 @@ va_status create_handle(const va_problem *pb_in, const va::KernelSet *given, va_
     alloc((void **)&h->n_acc, sizeof(int32_t) * B);
     alloc((void **)&h->n_rej, sizeof(int32_t) * B);
     alloc((void **)&h->status, sizeof(int32_t) * B);
-    alloc((void **)&h->counters, sizeof(int32_t) * 8);
+    alloc((void **)&h->counters, sizeof(int32_t) * VA_WORK_INTS);
     alloc((void **)&h->order, sizeof(int32_t) * (size_t)pb->batch);
     alloc((void **)&h->order_fwd, sizeof(int32_t) * (size_t)pb->batch);
     alloc((void **)&h->order_fwd_next, sizeof(int32_t) * (size_t)pb->batch);
-    alloc((void **)&h->order_tmp, sizeof(int32_t) * 2 * VA_ORDER_BUCKETS);
     if (pb->n_obs > 0 || h->obs_ckpt) {
         alloc((void **)&h->obs_row, sizeof(int32_t) * std::max<size_t>(1, (size_t)B * pb->n_obs));
         if (h->obs_ckpt) {
@@ -1261,7 +1325,7 @@ va_status create_handle(const va_problem *pb_in, const va::KernelSet *given, va_
         if (e == hipSuccess) e = hipEventCreateWithFlags(&h->ev_fwd, hipEventDisableTiming);
     }
     // no previous forward: zero attempt counts and no long instances
-    if (e == hipSuccess) e = hipMemset(h->counters, 0, sizeof(int32_t) * 8);
+    if (e == hipSuccess) e = hipMemset(h->counters, 0, sizeof(int32_t) * VA_WORK_INTS);
     if (e == hipSuccess) e = hipMemset(h->n_acc, 0, sizeof(int32_t) * B);
     if (e == hipSuccess) e = hipMemset(h->n_rej, 0, sizeof(int32_t) * B);
     {  // the first forward takes instances in index order
@@ -1314,10 +1378,14 @@ va_status va_forward(va_handle *h, double *y, const double *p, int32_t *n_accept
     if ((st = check_rows(h))) return st;
     if (!y || !p) return fail(VA_ERR_INVALID, "y and p are required");
     hipStream_t s = (hipStream_t)stream;
-    st = h->pb.mode == VA_MODE_PLAIN ? forward_plain(h, y, p, s) : forward_persistent(h, y, p, s);
-    if (st) return st;
+    const CountsOut out{n_accepted, n_rejected, lane_status};
+    if (h->pb.mode == VA_MODE_PLAIN) {
+        if ((st = forward_plain(h, y, p, s)) || (st = copy_out(h, out, s))) return st;
+    } else if ((st = forward_persistent(h, y, y, p, out, s))) {
+        return st;
+    }
     h->have_forward = true;
-    return copy_out(h, n_accepted, n_rejected, lane_status, s);
+    return VA_OK;
 }
 
 va_status va_adjoint(va_handle *h, const double *p, int32_t nout, double *lambda, double *mu,
@@ -1456,35 +1524,31 @@ static va_status solve_enqueue(va_handle *h, const double *y0, const double *p, 
     hipStream_t s = (hipStream_t)stream;
     const int64_t B = h->pb.batch;
     const int n = h->ks.n, np = h->ks.np;
-    const bool split = h->pb.mode != VA_MODE_PLAIN && split_solve(h);
-    if (split) {
-        // copies y0 and the counts itself
-        st = solve_split(h, y0, yT, p, cost, cost_weights, J, dJdy0, dJdp, n_accepted,
-                         n_rejected, lane_status, s);
-        if (!st) h->have_forward = true;
-        return st;
+    const CountsOut out{n_accepted, n_rejected, lane_status};
+    if (h->pb.mode != VA_MODE_PLAIN) {
+        if (split_solve(h)) {
+            st = solve_split(h, y0, yT, p, cost, cost_weights, J, dJdy0, dJdp, out, s);
+            if (!st) h->have_forward = true;
+            return st;
+        }
+        if ((st = forward_persistent(h, yT, y0, p, out, s))) return st;
+        h->have_forward = true;
+        return reverse_persistent(h, p, cost, cost_weights, yT, J, dJdy0, dJdp, 1, s, false, true);
     }
     if (yT != y0) {
         hipLaunchKernelGGL(k_copy_f64, dim3(blocks_for((int64_t)n * B, 256)), dim3(256), 0, s, yT,
                            y0, (int64_t)n * B);
         VA_HIP(hipGetLastError());
     }
-    if (h->pb.mode == VA_MODE_PLAIN) {
-        if ((st = forward_plain(h, yT, p, s))) return st;
-        h->have_forward = true;
-        VA_HIP(va::launch_plain_cost(cost, cost_weights, yT, J, dJdy0, h->status, B, n,
-                                     blocks_for(B, h->block), h->block, s));
-        if ((st = fill_f64(dJdp, 0.0, (int64_t)np * B, s))) return st;
-        int32_t smax = 0;
-        if ((st = read_max_steps(h, &smax, s))) return st;
-        if ((st = reverse_plain_seed(h, p, dJdy0, dJdp, smax, s))) return st;
-    } else {
-        if ((st = forward_persistent(h, yT, p, s))) return st;
-        h->have_forward = true;
-        if ((st = reverse_persistent(h, p, cost, cost_weights, yT, J, dJdy0, dJdp, 1, s)))
-            return st;
-    }
-    return copy_out(h, n_accepted, n_rejected, lane_status, s);
+    if ((st = forward_plain(h, yT, p, s))) return st;
+    h->have_forward = true;
+    VA_HIP(va::launch_plain_cost(cost, cost_weights, yT, J, dJdy0, h->status, B, n,
+                                 blocks_for(B, h->block), h->block, s));
+    if ((st = fill_f64(dJdp, 0.0, (int64_t)np * B, s))) return st;
+    int32_t smax = 0;
+    if ((st = read_max_steps(h, &smax, s))) return st;
+    if ((st = reverse_plain_seed(h, p, dJdy0, dJdp, smax, s))) return st;
+    return copy_out(h, out, s);
 }
 
 // Observation-kernel solve: the running cost over obs (K = pb.n_obs), plus the
@@ -1499,13 +1563,7 @@ static va_status observed_enqueue(va_handle *h, const double *y0, const double *
     va_status st = VA_OK;
     hipStream_t s = (hipStream_t)stream;
     const int64_t B = h->pb.batch;
-    const int n = h->ks.n;
-    if (yT != y0) {
-        hipLaunchKernelGGL(k_copy_f64, dim3(blocks_for((int64_t)n * B, 256)), dim3(256), 0, s, yT,
-                           y0, (int64_t)n * B);
-        VA_HIP(hipGetLastError());
-    }
-    if ((st = fill_i32(h->counters, 0, 4, s))) return st;
+    if ((st = clear_and_copy(h, yT, y0, s))) return st;
     va::ObsStore os;
     os.ckpt = h->obs_ckpt;
     os.traj = h->traj;
@@ -1538,8 +1596,9 @@ static va_status observed_enqueue(va_handle *h, const double *y0, const double *
     VA_HIP(h->ks.obs_fwd(f, blocks_for(std::min<int64_t>(h->lanes_obs_fwd, B), h->block),
                          h->block, s));
     h->have_forward = !h->obs_ckpt;
-    if (order_wanted(h, h->lanes_obs_fwd) && (st = order_by_length(h, 1, s))) return st;
-    if ((st = order_longest_first(h, s))) return st;
+    if ((st = build_orders(h, order_wanted(h, h->lanes_obs_fwd) ? 3 : 1, false,
+                           CountsOut{n_accepted, n_rejected, lane_status}, s)))
+        return st;
     va::ObsRevArgs r;
     r.sp = f.sp;
     r.p = p;
@@ -1559,7 +1618,7 @@ static va_status observed_enqueue(va_handle *h, const double *y0, const double *
     r.st = os;
     VA_HIP(h->ks.obs_rev(r, blocks_for(std::min<int64_t>(h->lanes_obs_rev, B), h->block),
                          h->block, s));
-    return copy_out(h, n_accepted, n_rejected, lane_status, s);
+    return VA_OK;
 }
 
 va_status va_solve_observed(va_handle *h, const double *y0, const double *p, const double *obs_t,
@@ -1596,12 +1655,7 @@ va_status va_solve_shared(va_handle *h, const double *y0, const double *p, const
     hipStream_t s = (hipStream_t)stream;
     const int64_t B = h->pb.batch;
     const int n = h->ks.n;
-    if (yT != y0) {
-        hipLaunchKernelGGL(k_copy_f64, dim3(blocks_for((int64_t)n * B, 256)), dim3(256), 0, s, yT,
-                           y0, (int64_t)n * B);
-        VA_HIP(hipGetLastError());
-    }
-    if ((st = fill_i32(h->counters, 0, 4, s))) return st;
+    if ((st = clear_and_copy(h, yT, y0, s))) return st;
     va::SharedFwdArgs f;
     f.sp = solve_params(h);
     f.y = yT;
@@ -1617,7 +1671,8 @@ va_status va_solve_shared(va_handle *h, const double *y0, const double *p, const
     // J and the seed dJ/dy(T), written into dJdy0 and swept back in place
     VA_HIP(va::launch_plain_cost(cost, cost_w, yT, J, dJdy0, h->status, B, n, blocks_for(B, 256),
                                  256, s));
-    if ((st = order_longest_first(h, s))) return st;
+    if ((st = build_orders(h, 1, false, CountsOut{n_accepted, n_rejected, lane_status}, s)))
+        return st;
     va::SharedRevArgs r;
     r.sp = f.sp;
     r.r = p;
@@ -1633,7 +1688,7 @@ va_status va_solve_shared(va_handle *h, const double *y0, const double *p, const
     r.gscr = h->shared_gscr;
     VA_HIP(h->ks.shared_rev(r, h->shared_grid, s));
     VA_HIP(va::launch_glvs_reduce(h->abar_part, h->shared_grid, dJdp_shared, s));
-    return copy_out(h, n_accepted, n_rejected, lane_status, s);
+    return VA_OK;
 }
 
 va_status va_trajectory(va_handle *h, int64_t instance, double *rows, int64_t max_rows,
@@ -1960,8 +2015,8 @@ va_status va_solve_noalloc(const va_problem *pb, const double *y0, const double 
             return st;
     }
     if (n_accepted || n_rejected || lane_status) {
-        hipLaunchKernelGGL(k_copy_counts, dim3(blocks_for(B, 256)), dim3(256), 0, s, n_accepted,
-                           n_rejected, lane_status, nacc, nrej, stat, B);
+        hipLaunchKernelGGL(k_copy_counts, dim3(blocks_for(B, 256)), dim3(256), 0, s,
+                           CountsOut{n_accepted, n_rejected, lane_status}, nacc, nrej, stat, B);
         VA_HIP(hipGetLastError());
     }
     return VA_OK;
