@@ -253,6 +253,7 @@ struct OrderArgs {
     int64_t B;
     int modes;       // bit 0: the reverse order, bit 1: the forward order
     int items;       // instances per thread, at most VA_ORDER_ITEMS
+    const int32_t *from;  // the scatter takes instances in this order (null: index order)
     int32_t *work;   // per mode a histogram and cursors, cleared before
     int32_t *order[2], *n_long[2];
 };
@@ -307,12 +308,13 @@ __global__ void __launch_bounds__(VA_ORDER_BUCKETS) k_order_scatter(OrderArgs a)
         }
         if (blockIdx.x == 0 && k == VA_LONG_BUCKET)
             *a.n_long[m] = sfx[k] < VA_LONG_MAX ? sfx[k] : VA_LONG_MAX;
-        int bucket[VA_ORDER_ITEMS], rank[VA_ORDER_ITEMS];
+        int bucket[VA_ORDER_ITEMS], rank[VA_ORDER_ITEMS], inst[VA_ORDER_ITEMS];
 #pragma unroll
         for (int j = 0; j < VA_ORDER_ITEMS; ++j) {
             const int64_t b = b0 + (int64_t)j * VA_ORDER_BUCKETS;
             if (j < a.items && b < a.B) {
-                bucket[j] = order_bucket(a.n_acc, a.n_rej, a.status, b, m);
+                inst[j] = a.from ? a.from[b] : (int32_t)b;
+                bucket[j] = order_bucket(a.n_acc, a.n_rej, a.status, inst[j], m);
                 rank[j] = atomicAdd(&cnt[bucket[j]], 1);
             }
         }
@@ -323,7 +325,7 @@ __global__ void __launch_bounds__(VA_ORDER_BUCKETS) k_order_scatter(OrderArgs a)
 #pragma unroll
         for (int j = 0; j < VA_ORDER_ITEMS; ++j) {
             const int64_t b = b0 + (int64_t)j * VA_ORDER_BUCKETS;
-            if (j < a.items && b < a.B) a.order[m][sfx[bucket[j]] + rank[j]] = (int32_t)b;
+            if (j < a.items && b < a.B) a.order[m][sfx[bucket[j]] + rank[j]] = inst[j];
         }
         __syncthreads();
     }
@@ -332,8 +334,8 @@ __global__ void __launch_bounds__(VA_ORDER_BUCKETS) k_order_scatter(OrderArgs a)
 // Digest of each instance's stored step sequence: d = 0x9E3779B97F4A7C15, then for
 // every stored point n = 0..n_acc: d = mix(d ^ bits(t_n)); d = mix(d ^ bits(h_n)),
 // mix the SplitMix64 finaliser (the oracle's orc_step_digest).  0 for instances
-// whose forward did not end OK.  plain: rows [row][field][instance], else
-// [instance][row][field] with `fields` doubles per row.
+// whose forward did not end OK.  plain: rows [row][field][instance], else in the
+// handle's row layout with `fields` doubles per row.
 __device__ __forceinline__ uint64_t digest_mix(uint64_t z)
 {
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
@@ -341,7 +343,26 @@ __device__ __forceinline__ uint64_t digest_mix(uint64_t z)
     return z ^ (z >> 31);
 }
 
-__global__ void __launch_bounds__(256) k_step_digest(const double *traj, int64_t B, int64_t cap,
+// Offset of row k of instance b in a persistent store of `fields` doubles per row.
+__device__ __forceinline__ int64_t persistent_row(const va::RowLayout &l, const int32_t *slot,
+                                                  int64_t b, int64_t k, int fields)
+{
+    const int64_t s = slot ? slot[b] : b;
+    return (s / va::VA_ROW_TILE) * l.tile + (s % va::VA_ROW_TILE) * l.lane +
+           (k / va::VA_ROW_BLOCK) * l.blk + (k % va::VA_ROW_BLOCK) * fields;
+}
+
+// Rows 0 .. nrows - 1 of instance b, one after the other.
+__global__ void k_gather_persistent(const double *traj, va::RowLayout l, const int32_t *slot,
+                                    int64_t b, int fields, int64_t nrows, double *out)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nrows * fields) return;
+    out[i] = traj[persistent_row(l, slot, b, i / fields, fields) + i % fields];
+}
+
+__global__ void __launch_bounds__(256) k_step_digest(const double *traj, va::RowLayout l,
+                                                     const int32_t *slot, int64_t B, int64_t cap,
                                                      int fields, int plain, const int32_t *n_acc,
                                                      const int32_t *status, uint64_t *out)
 {
@@ -357,7 +378,7 @@ __global__ void __launch_bounds__(256) k_step_digest(const double *traj, int64_t
                 t = traj[((size_t)k * fields) * (size_t)B + b];
                 hs = traj[((size_t)k * fields + 1) * (size_t)B + b];
             } else {
-                const double *r = traj + ((size_t)b * (size_t)(cap + 1) + (size_t)k) * fields;
+                const double *r = traj + persistent_row(l, slot, b, k, fields);
                 t = r[0];
                 hs = r[1];
             }
@@ -379,8 +400,10 @@ struct va_handle {
     int cu_count = 0;
     int block = 256;
     int64_t lanes_fwd = 0, lanes_rev = 0;  // instances in flight of the persistent kernels
-    // persistent store
+    // persistent store and its row layout; slot [B] is null where instance b is slot b
     double *traj = nullptr;
+    va::RowLayout rows;
+    int32_t *slot = nullptr;
     // plain store + state
     double *ptraj = nullptr, *pl_t = nullptr, *pl_dt = nullptr, *pl_k0 = nullptr,
            *pl_pbar = nullptr;
@@ -489,6 +512,7 @@ void release(va_handle *h)
 {
     if (!h) return;
     hipFree(h->traj);
+    hipFree(h->slot);
     hipFree(h->ptraj);
     hipFree(h->pl_t);
     hipFree(h->pl_dt);
@@ -534,8 +558,10 @@ va_status clear_and_copy(va_handle *h, double *yT, const double *y0, hipStream_t
 // forward (its prologue cleared the histograms), with the caller's counts copied:
 // bit 0 of modes into h->order (the reverse, by accepted steps), bit 1 into
 // h->order_fwd (the next forward, by attempts) or, with next, into
-// h->order_fwd_next, each with its count of long instances.
-va_status build_orders(va_handle *h, int modes, bool next, const CountsOut &out, hipStream_t s)
+// h->order_fwd_next, each with its count of long instances.  from: the order the
+// forward took (with next only: it may be h->order_fwd), kept within a bucket.
+va_status build_orders(va_handle *h, int modes, bool next, const CountsOut &out, hipStream_t s,
+                       const int32_t *from = nullptr)
 {
     OrderArgs a;
     a.n_acc = h->n_acc;
@@ -543,6 +569,7 @@ va_status build_orders(va_handle *h, int modes, bool next, const CountsOut &out,
     a.status = h->status;
     a.B = h->pb.batch;
     a.modes = modes;
+    a.from = from;
     a.items = (int)std::min<int64_t>(VA_ORDER_ITEMS, std::max<int64_t>(1, a.B >> 14));
     a.work = h->counters + VA_COUNTERS;
     a.order[0] = h->order;
@@ -554,6 +581,22 @@ va_status build_orders(va_handle *h, int modes, bool next, const CountsOut &out,
     hipLaunchKernelGGL(k_order_hist, dim3(grid), dim3(VA_ORDER_BUCKETS), 0, s, a, out);
     hipLaunchKernelGGL(k_order_scatter, dim3(grid), dim3(VA_ORDER_BUCKETS), 0, s, a);
     VA_HIP(hipGetLastError());
+    return VA_OK;
+}
+
+// The orders after a forward of the one-lane kernels that took instances in the
+// order `taken`: neighbours of that order, whose rows are neighbours, stay
+// together in the reverse's.  A recorded solve, whose replays share one buffer,
+// rebuilds the forward order in place and keeps neighbours by index.
+va_status orders_after(va_handle *h, int modes, const int32_t *taken, const CountsOut &out,
+                       hipStream_t s)
+{
+    if (h->capturing || !taken) return build_orders(h, modes, false, out, s);
+    if (va_status st = build_orders(h, modes, true, out, s, taken)) return st;
+    if (modes & 2) {
+        std::swap(h->order_fwd, h->order_fwd_next);
+        h->nlong_idx = 11 - h->nlong_idx;
+    }
     return VA_OK;
 }
 
@@ -723,6 +766,8 @@ va_status forward_persistent(va_handle *h, double *y, const double *y0, const do
     a.status = h->status;
     a.counter = h->counters + 0;
     a.max_steps_seen = h->counters + 2;
+    a.rows = h->rows;
+    a.slot = h->slot;
     const bool reuse = reuse_order(h, h->lanes_fwd);
     a.order = reuse ? h->order_fwd : nullptr;
     const int64_t lanes = std::min<int64_t>(h->lanes_fwd, B);
@@ -743,7 +788,8 @@ va_status forward_persistent(va_handle *h, double *y, const double *y0, const do
         VA_HIP(h->ks.fwd(a, blocks_for(lanes, h->ks.slots(h->block)), h->block, s));
     }
     const int modes = (order_wanted(h, h->lanes_fwd) ? 2 : 0) | (split_reverse(h) ? 0 : 1);
-    return build_orders(h, modes, false, out, s);
+    return h->ks.layout == 0 ? orders_after(h, modes, a.order, out, s)
+                             : build_orders(h, modes, false, out, s);
 }
 
 // Seeds a work item of a reverse of nout seeds takes.  The Lotka-Volterra groups
@@ -790,6 +836,8 @@ va_status reverse_persistent(va_handle *h, const double *p, int cost, const doub
     a.counter = h->counters + 1;
     a.seeds_per_item = cost ? 0 : seeds_per_item(h, nout);
     a.identity = identity ? 1 : 0;
+    a.rows = h->rows;
+    a.slot = h->slot;
     const bool im = instance_major(h);
     const bool add = cost == 0 && !identity;
     const int nseed = cost ? 1 : nout;
@@ -1108,6 +1156,12 @@ TuneKey tune_key(const va_problem *pb, int device)
     return TuneKey{device, pb->system, pb->n_state, pb->tableau, pb->adaptive, pb->n_obs, bucket};
 }
 
+// Instances from which a one-lane store is tiled: below, the rows of a few waves are
+// in reach of the translation caches however they lie, and a lone wave's reverse
+// was slower on tiles (Van der Pol, B=1024: reverse 0.78 ms instance-major, 0.86
+// tiled; RK4 oscillator, B=40000: solve 1.16 ms instance-major, 1.04 tiled).
+constexpr int64_t VA_TILED_MIN = 4096;
+
 va_status create_handle(const va_problem *pb_in, const va::KernelSet *given, va_handle **out)
 {
     g_err[0] = 0;
@@ -1290,7 +1344,20 @@ va_status create_handle(const va_problem *pb_in, const va::KernelSet *given, va_
                                             ks.shared_waves * 2 * ks.s_rev * 64 * 4);
     }
     if (pb->mode == VA_MODE_PERSISTENT) {
-        if (full_store) alloc((void **)&h->traj, sizeof(double) * rows * (size_t)B * (ks.n + 2));
+        if (full_store) {
+            // one-lane kernels that know tiled rows have them in large stores, the
+            // others instance-major
+            const int F = ks.n + 2;
+            if (ks.layout == 0 && ks.table_version >= 2 && B >= VA_TILED_MIN) {
+                h->rows = va::rows_tiled(pb->max_steps, F);
+                const size_t tiles = ((size_t)B + va::VA_ROW_TILE - 1) / va::VA_ROW_TILE;
+                alloc((void **)&h->traj, sizeof(double) * tiles * (size_t)h->rows.tile);
+                alloc((void **)&h->slot, sizeof(int32_t) * (size_t)B);
+            } else {
+                h->rows = va::rows_instance_major(pb->max_steps, F);
+                alloc((void **)&h->traj, sizeof(double) * rows * (size_t)B * F);
+            }
+        }
         if (ks.layout == 1 && full_store) {
             // instance-major parameters and dJ/dp sums of the row kernels
             alloc((void **)&h->pim, sizeof(double) * (size_t)B * ks.np);
@@ -1567,6 +1634,8 @@ static va_status observed_enqueue(va_handle *h, const double *y0, const double *
     va::ObsStore os;
     os.ckpt = h->obs_ckpt;
     os.traj = h->traj;
+    os.rows = h->rows;
+    os.slot = h->slot;
     os.ck = h->obs_ck;
     os.slots = h->obs_slots;
     os.stride_max = h->obs_stride_max;
@@ -1596,7 +1665,7 @@ static va_status observed_enqueue(va_handle *h, const double *y0, const double *
     VA_HIP(h->ks.obs_fwd(f, blocks_for(std::min<int64_t>(h->lanes_obs_fwd, B), h->block),
                          h->block, s));
     h->have_forward = !h->obs_ckpt;
-    if ((st = build_orders(h, order_wanted(h, h->lanes_obs_fwd) ? 3 : 1, false,
+    if ((st = orders_after(h, order_wanted(h, h->lanes_obs_fwd) ? 3 : 1, f.order,
                            CountsOut{n_accepted, n_rejected, lane_status}, s)))
         return st;
     va::ObsRevArgs r;
@@ -1713,15 +1782,20 @@ va_status va_trajectory(va_handle *h, int64_t instance, double *rows, int64_t ma
     if (ncopy <= 0) return VA_OK;
     const int n = h->ks.n;
     const size_t bytes = sizeof(double) * (size_t)ncopy * (n + 2);
-    if (h->pb.mode == VA_MODE_PERSISTENT) {
+    if (h->pb.mode == VA_MODE_PERSISTENT && !h->slot) {
         const double *src = h->traj + (size_t)instance * (size_t)(h->pb.max_steps + 1) * (n + 2);
         VA_HIP(hipMemcpyAsync(rows, src, bytes, hipMemcpyDeviceToHost, s));
     } else {
         double *tmp = nullptr;
         VA_HIP(hipMallocAsync((void **)&tmp, bytes, s));
         const int fields = 2 + n;
-        hipLaunchKernelGGL(k_gather_rows, dim3(blocks_for(ncopy * (n + 2), 256)), dim3(256), 0, s,
-                           h->ptraj, instance, h->pb.batch, fields, n, ncopy, tmp);
+        const dim3 grid(blocks_for(ncopy * fields, 256));
+        if (h->slot)
+            hipLaunchKernelGGL(k_gather_persistent, grid, dim3(256), 0, s, h->traj, h->rows,
+                               h->slot, instance, fields, ncopy, tmp);
+        else
+            hipLaunchKernelGGL(k_gather_rows, grid, dim3(256), 0, s, h->ptraj, instance,
+                               h->pb.batch, fields, n, ncopy, tmp);
         hipError_t e = hipMemcpyAsync(rows, tmp, bytes, hipMemcpyDeviceToHost, s);
         hipFreeAsync(tmp, s);
         VA_HIP(e);
@@ -1993,8 +2067,10 @@ va_status va_solve_noalloc(const va_problem *pb, const double *y0, const double 
     a.status = stat;
     a.counter = counters + 0;
     a.max_steps_seen = counters + 2;
+    a.rows = va::rows_instance_major(pb->max_steps, n + 2);
     VA_HIP(ks.fwd(a, blocks_for(lanes_f, per_block), block, s));
     va::RevArgs r{};
+    r.rows = a.rows;
     r.sp = sp;
     r.order = nullptr;
     r.p = im ? pim : p;
@@ -2035,7 +2111,8 @@ va_status va_step_digest(va_handle *h, uint64_t *digest, void *stream)
     const int64_t B = h->pb.batch;
     const bool plain = h->pb.mode == VA_MODE_PLAIN;
     hipLaunchKernelGGL(k_step_digest, dim3(blocks_for(B, 256)), dim3(256), 0, s,
-                       plain ? h->ptraj : h->traj, B, (int64_t)h->pb.max_steps, h->ks.n + 2,
+                       plain ? h->ptraj : h->traj, h->rows, h->slot, B,
+                       (int64_t)h->pb.max_steps, h->ks.n + 2,
                        plain ? 1 : 0, h->n_acc, h->status, digest);
     VA_HIP(hipGetLastError());
     return VA_OK;

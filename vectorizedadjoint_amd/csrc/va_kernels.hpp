@@ -14,6 +14,33 @@ struct SolveParams {
     int32_t adaptive;
 };
 
+// Where the one-lane kernels keep an instance's rows (t, h, y), F = N + 2 doubles
+// each: row r of storage slot s at traj[(s / 64) tile + (s % 64) lane +
+// (r / 4) blk + (r % 4) F].  A handle's store is tiled: four rows of a slot lie
+// together (128 bytes for N = 2, a cache line), beside those of the 63 other
+// slots of its tile, and a forward stores the k-th instance it takes in slot k
+// (slot[b] = k), so the lanes of a wave write one 8 KB block after another.
+// With rows instance-major each lane was at an address of its own in a store of
+// tens of GB, and address translation bound both sweeps (solve of the oscillator,
+// B=2^20: 26.4 ms; tiled, and by the lines of k_fwd and k_rev_lines, 19.2 ms).
+// slot == null: slot b is instance b's.
+struct RowLayout {
+    int64_t tile = 0, lane = 0, blk = 0;
+};
+constexpr int VA_ROW_TILE = 64, VA_ROW_BLOCK = 4;
+
+// Rows instance-major, [B][cap + 1][F].
+inline RowLayout rows_instance_major(int64_t cap, int F)
+{
+    return RowLayout{VA_ROW_TILE * (cap + 1) * F, (cap + 1) * F, VA_ROW_BLOCK * F};
+}
+inline int64_t row_blocks(int64_t cap) { return (cap + VA_ROW_BLOCK) / VA_ROW_BLOCK; }
+inline RowLayout rows_tiled(int64_t cap, int F)
+{
+    const int64_t blk = (int64_t)VA_ROW_TILE * VA_ROW_BLOCK * F;
+    return RowLayout{blk * row_blocks(cap), VA_ROW_BLOCK * F, blk};
+}
+
 // Persistent forward: each lane takes instances from *counter until B is reached.
 struct FwdArgs {
     SolveParams sp;
@@ -26,6 +53,8 @@ struct FwdArgs {
     const int32_t *order = nullptr;  // [B] or null: the k-th instance taken is order[k]
     const int32_t *split = nullptr;  // null: queue positions [0, B); else part 0 takes
     int32_t part = 0;                // [0, *split), part 1 takes [*split, B)
+    RowLayout rows;                  // one-lane kernels
+    int32_t *slot = nullptr;         // [B] or null, written
 };
 
 // Persistent reverse over the stored trajectory.
@@ -59,6 +88,8 @@ struct RevArgs {
     // (cost == 0) the seeds are the unit vectors (nout = N): lambda is neither read
     // nor written, and mu = 0.0 + sum
     int32_t identity = 0;
+    RowLayout rows;                  // one-lane kernels
+    const int32_t *slot = nullptr;   // [B] or null
 };
 
 // The work items of a reverse: groups of seeds per instance.
@@ -127,6 +158,8 @@ struct ObsStore {
     int32_t seg_rows = 0;  // rows of the per-lane row buffer (stride_max with one level)
     int32_t slots2 = 0;    // level-2 checkpoints per lane
     double *ck2 = nullptr; // [lanes][slots2][N+3], lanes interleaved like seg
+    RowLayout rows;        // of traj
+    int32_t *slot = nullptr;
 };
 
 struct ObsFwdArgs {
@@ -189,9 +222,10 @@ struct SharedRevArgs {
 
 // Layout version of KernelSet: kernel tables made in a caller's translation unit
 // (VA_DEVICE_SYSTEM) are accepted with the library's size and a version it knows.
-// Version 2 kernels read RevArgs::seeds_per_item and identity; version 1 kernels
-// (the same table and argument layout up to those members) sweep all seeds of an
-// instance one after the other and are never given either.
+// Version 2 kernels read RevArgs::seeds_per_item, identity and the rows and slot
+// members; version 1 kernels (the same table and argument layout up to those
+// members) sweep all seeds of an instance one after the other, keep their rows
+// instance-major, and are never given any of them.
 constexpr int32_t VA_KERNEL_TABLE_VERSION = 2;
 constexpr int32_t VA_KERNEL_TABLE_OLDEST = 1;
 

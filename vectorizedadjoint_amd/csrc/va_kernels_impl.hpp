@@ -33,6 +33,36 @@ enum { COST_REFERENCE = 0, COST_SUM = 1, COST_SQUARED_NORM = 2, COST_LINEAR = 3 
 // encoding: vmcnt 0, expcnt and lgkmcnt left at their maxima.)
 __device__ __forceinline__ void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
+// Slot s's rows, and row r among them (see RowLayout).
+__device__ __forceinline__ int64_t slot_rows(const RowLayout &l, int64_t s)
+{
+    return (int64_t)((uint64_t)s / VA_ROW_TILE) * l.tile + (int64_t)(s & (VA_ROW_TILE - 1)) * l.lane;
+}
+template <int F>
+__device__ __forceinline__ int64_t row_offset(const RowLayout &l, int32_t r)
+{
+    const uint32_t u = (uint32_t)r;
+    return (int64_t)(u / VA_ROW_BLOCK) * l.blk + (u % VA_ROW_BLOCK) * F;
+}
+
+// A reverse's rows: (h, y) of row r of one slot, row 0 below it.  Five vector
+// instructions of address per row, for a lone wave pays for each of them.
+template <int F>
+struct RowsBack {
+    const double *p;   // the slot's row 0; always a slot of the store, also without an item
+    uint32_t blk = 0;  // bytes between blocks of rows
+    template <int N>
+    __device__ __forceinline__ void load(int32_t r, double &h, double (&y)[N]) const
+    {
+        const uint32_t u = r > 0 ? (uint32_t)r : 0u;
+        const char *at = (const char *)p + (uint64_t)(u / VA_ROW_BLOCK) * blk;
+        const double *q = (const double *)(at + (uint64_t)(u % VA_ROW_BLOCK * (F * 8)));
+        h = q[1];
+#pragma unroll
+        for (int i = 0; i < N; ++i) y[i] = q[2 + i];
+    }
+};
+
 template <int N>
 __device__ __forceinline__ bool all_finite(const double *y)
 {
@@ -41,6 +71,51 @@ __device__ __forceinline__ bool all_finite(const double *y)
     for (int i = 0; i < N; ++i) ok = ok && (fabs(y[i]) <= 1.7976931348623157e308);
     return ok;
 }
+
+// A wave's lines of four rows (N = 2, 128 bytes) on their way to or from the
+// tiled store, each lane's in LDS.  The stride of 144 bytes leaves the lanes'
+// 16-byte accesses, and the wave's accesses to eight lines at a time, without
+// bank conflicts.  Every lane of the wave calls store() and load().
+typedef double d2 __attribute__((ext_vector_type(2)));
+
+struct WaveLines {
+    d2 line[64][9];
+    d2 *addr[64];
+    int src[64];
+
+    // Write the lines of the lanes with full set to to[] of each.
+    __device__ __forceinline__ void store(bool full, int lane, double *to)
+    {
+        const uint64_t m = __builtin_amdgcn_ballot_w64(full);
+        if (m == 0) return;
+        const int n = __builtin_popcountll(m);
+        const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                   __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+        if (full) {
+            addr[rank] = reinterpret_cast<d2 *>(to);
+            src[rank] = lane;
+        }
+        __builtin_amdgcn_wave_barrier();
+        for (int j = lane >> 3; j < n; j += 8) addr[j][lane & 7] = line[src[j]][lane & 7];
+        __builtin_amdgcn_wave_barrier();
+    }
+
+    // Chunk lane % 8 of the lines of lanes lane / 8 + 8 j, at from[] of each.
+    __device__ __forceinline__ void load(int lane, const double *from, d2 (&v)[8])
+    {
+        addr[lane] = const_cast<d2 *>(reinterpret_cast<const d2 *>(from));
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = addr[(lane >> 3) + 8 * j][lane & 7];
+        __builtin_amdgcn_wave_barrier();
+    }
+    __device__ __forceinline__ void keep(int lane, const d2 (&v)[8])
+    {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) line[(lane >> 3) + 8 * j][lane & 7] = v[j];
+        __builtin_amdgcn_wave_barrier();
+    }
+};
 
 // ---------------------------------------------------------------------------
 // Persistent forward
@@ -54,10 +129,21 @@ __device__ __forceinline__ bool all_finite(const double *y)
 // (With the waits on each step's stores and rows, here and in k_rev: solve of
 // Van der Pol, B=1024, 2.67 ms, oscillator, B=2^20, 49.2 ms; without 2.10 and
 // 34.4; with selects in the step control and, for Lone, the constants in vector
-// registers 1.83 and 33.8.)
-template <class Sys, class Tab, bool Adaptive, bool Lone>
+// registers 1.83 and 33.8; with rows three ahead in k_rev's Lone loop 1.73.)
+//
+// Lines (N = 2, tiled rows): a row's two 16-byte stores touch a line per lane
+// each, and at 128 requests per row of a wave the path to L2 was the bound of a
+// full chip (oscillator, B=2^20: forward 14.4 ms, 6.4 of them vector
+// instructions).  A lane there gathers its line, four rows, in LDS; lanes whose
+// lines are full hand them to the whole wave, which stores eight lines per
+// instruction: forward 11.2 ms.
+template <class Sys, class Tab, bool Adaptive, bool Lone, bool Lines = false>
 __global__ void __launch_bounds__(256) k_fwd(FwdArgs a)
 {
+    static_assert(!Lines || Sys::N == 2, "lines of four rows are 128 bytes for N = 2");
+    __shared__ WaveLines lines[Lines ? 4 : 1];
+    const int lane = threadIdx.x & 63;
+    WaveLines &wl = lines[Lines ? threadIdx.x >> 6 : 0];
     if constexpr (Adaptive) load_ctrl_tables();
     constexpr int N = Sys::N;
     constexpr int F = N + 2;  // row (t_n, h_n, y_n)
@@ -73,8 +159,9 @@ __global__ void __launch_bounds__(256) k_fwd(FwdArgs a)
     double t = 0.0, dt = 0.0;
     int64_t b = 0;
     int32_t count = 0, rej = 0, tries = 0, st = LANE_OK;
-    bool need = true;
-    double *row = nullptr;  // row `count` of the instance
+    bool need = true, over = false;  // over (Lines): no instance left for this lane
+    double *row = nullptr;  // row `count` of the instance (Lines: the first of its block)
+    const int64_t row_wrap = a.rows.blk - (VA_ROW_BLOCK - 1) * F;  // to the next block of rows
 
     // The head of the controlled loop at the point (t, y): false when the instance
     // is done (or has no room for another step), else dt clipped to end at t1.
@@ -88,67 +175,101 @@ __global__ void __launch_bounds__(256) k_fwd(FwdArgs a)
         tries = 0;
         return more && count < cap;
     };
-    auto store_row = [&](double h) {
-        row[0] = t;
-        row[1] = h;
+    auto put_row = [&](double *to, double h) {
+        to[0] = t;
+        to[1] = h;
 #pragma unroll
-        for (int i = 0; i < N; ++i) row[2 + i] = y[i];
+        for (int i = 0; i < N; ++i) to[2 + i] = y[i];
+    };
+    auto store_row = [&](double h) {
+        if constexpr (Lines)
+            put_row(reinterpret_cast<double *>(wl.line[lane] + 2 * (count % VA_ROW_BLOCK)), h);
+        else
+            put_row(row, h);
+    };
+
+    // one attempt, and after an accepted one the head of the next step
+    auto attempt = [&](bool &finish, bool &full) {
+        const double h = Adaptive ? dt : sp.dt0;
+        double K[Tab::SF][N], ynew[N], xerr[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) K[0][i] = k0[i];
+        R::attempt(tc, q, y, K, h, ynew, xerr);
+        bool accept = true, fail = false;
+        if constexpr (Adaptive) {
+            const double err = R::error_norm(sp.atol, sp.rtol, h, y, k0, xerr);
+            accept = control_step<Tab>(h, err, dt, pc);
+            fail = ++tries > sp.max_attempts;
+        }
+        if (accept) {
+            const double tn = Adaptive ? t + h : sp.t0 + (double)(count + 1) * sp.dt0;
+            store_row(stored_step(tn, t));
+            ++count;
+            full = count % VA_ROW_BLOCK == 0;
+            if constexpr (!Lines) row += full ? row_wrap : F;
+            t = tn;
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                y[i] = ynew[i];
+                if constexpr (Tab::FSAL) k0[i] = K[Tab::SF - 1][i];
+            }
+            finish = !begin_step();
+        } else {
+            ++rej;
+        }
+        if (fail) {
+            st = LANE_MAX_FAIL;
+            finish = true;
+        }
     };
 
     for (;;) {
-        bool finish = false;
-        if (need) {
-            b = atomicAdd(a.counter, 1);
-            if (b >= B) break;
-            if (a.order) b = a.order[b];
-            Sys::load(q, a.p, B, b, sp.kconst);
-#pragma unroll
-            for (int i = 0; i < N; ++i) y[i] = a.y[(int64_t)i * B + b];
-            t = sp.t0;
-            dt = sp.dt0;
-            count = rej = 0;
-            st = LANE_OK;
-            need = false;
-            row = a.traj + (size_t)b * (size_t)(sp.cap + 1) * F;
-            wait_vmem();
-            if constexpr (Tab::FSAL) Sys::rhs(q, y, k0);
-            finish = !begin_step();
-        }
-        if (!finish) {
-            const double h = Adaptive ? dt : sp.dt0;
-            double K[Tab::SF][N], ynew[N], xerr[N];
-#pragma unroll
-            for (int i = 0; i < N; ++i) K[0][i] = k0[i];
-            R::attempt(tc, q, y, K, h, ynew, xerr);
-            bool accept = true, fail = false;
-            if constexpr (Adaptive) {
-                const double err = R::error_norm(sp.atol, sp.rtol, h, y, k0, xerr);
-                accept = control_step<Tab>(h, err, dt, pc);
-                fail = ++tries > sp.max_attempts;
-            }
-            if (accept) {
-                ++count;
-                const double tn = Adaptive ? t + h : sp.t0 + (double)count * sp.dt0;
-                store_row(stored_step(tn, t));
-                row += F;
-                t = tn;
-#pragma unroll
-                for (int i = 0; i < N; ++i) {
-                    y[i] = ynew[i];
-                    if constexpr (Tab::FSAL) k0[i] = K[Tab::SF - 1][i];
-                }
-                finish = !begin_step();
+        bool finish = false, full = false;
+        if (need && !over) {
+            const int64_t k = atomicAdd(a.counter, 1);
+            if constexpr (Lines) {
+                over = k >= B;
             } else {
-                ++rej;
+                if (k >= B) break;
             }
-            if (fail) {
-                st = LANE_MAX_FAIL;
-                finish = true;
+            if (!over) {
+                b = a.order ? a.order[k] : k;
+                if (a.slot) a.slot[b] = (int32_t)k;
+                Sys::load(q, a.p, B, b, sp.kconst);
+#pragma unroll
+                for (int i = 0; i < N; ++i) y[i] = a.y[(int64_t)i * B + b];
+                t = sp.t0;
+                dt = sp.dt0;
+                count = rej = 0;
+                st = LANE_OK;
+                need = false;
+                row = a.traj + slot_rows(a.rows, a.slot ? k : b);
+                wait_vmem();
+                if constexpr (Tab::FSAL) Sys::rhs(q, y, k0);
+                finish = !begin_step();
             }
+        }
+        if constexpr (Lines)
+            if (__builtin_amdgcn_ballot_w64(!over) == 0) break;  // the wave, all at once
+        if constexpr (Lone) {
+            // (a lone wave has an instance per lane: no lane waits for another's refill)
+            while (!finish) attempt(finish, full);
+        } else if (!finish && !over) {
+            attempt(finish, full);
+        }
+        if constexpr (Lines) {
+            wl.store(full, lane, row);
+            if (full) row += a.rows.blk;
         }
         if (finish) {
+            if constexpr (Lines) {  // the rows of a line that is not full
+                const d2 *l = wl.line[lane];
+                for (int r = 0; r < 2 * (count % VA_ROW_BLOCK); ++r)
+                    reinterpret_cast<d2 *>(row)[r] = l[r];
+                row += count % VA_ROW_BLOCK * F;
+            }
             if (st == LANE_OK) {
-                store_row(0.0);
+                put_row(row, 0.0);
                 if (!all_finite<N>(y)) st = LANE_NONFINITE;
             }
 #pragma unroll
@@ -246,6 +367,10 @@ __device__ __forceinline__ double terminal_cost(int cost, const double *w, const
 // its own, with many a lane takes NS seeds through one sweep, which recomputes the
 // stages once for all of them (RK4 oscillator, B=40000, two seeds, reverse alone
 // 1.16 ms one after the other).
+// Rows are loaded two steps ahead; for waves that run alone three steps share a
+// trip, so that no row is copied between registers and the wait for it lies where
+// it is used (Van der Pol, B=1024, reverse 0.78 ms with a copy and a wait per step,
+// 0.69 so).
 // ---------------------------------------------------------------------------
 template <class Sys, class Tab, bool Lone, int NS>
 __global__ void __launch_bounds__(256) k_rev(RevArgs a)
@@ -262,17 +387,11 @@ __global__ void __launch_bounds__(256) k_rev(RevArgs a)
     int64_t b = 0;
     int32_t o = 0, o_end = 0, n = -1;  // seeds o .. o + NS - 1, of those below o_end
     bool need = true;
-    const double *rows = nullptr;
-    // rows n and n - 1 of the sweep, each loaded two steps before its own, so that
-    // no step waits for memory (a step of a small system takes about 0.5 us, less
-    // than a read from HBM)
-    double h0 = 0.0, h1 = 0.0, y0[N] = {}, y1[N] = {};
-    auto load_row = [&](int32_t k, double &h, double (&y)[N]) {
-        const double *r = rows + (size_t)(k > 0 ? k : 0) * F;
-        h = r[1];
-#pragma unroll
-        for (int i = 0; i < N; ++i) y[i] = r[2 + i];
-    };
+    // the rows of the next steps, each loaded two steps before its own, so that no
+    // step waits for memory (a step of a small system takes about 0.6 us, less than
+    // a read from HBM)
+    double hr[3] = {}, yr[3][N] = {};
+    RowsBack<F> rows{a.traj, (uint32_t)a.rows.blk * 8u};
     // the seeds from o on, from the instance's last step
     auto start_sweep = [&]() {
         if (!a.cost) {
@@ -289,9 +408,19 @@ __global__ void __launch_bounds__(256) k_rev(RevArgs a)
 #pragma unroll
             for (int k = 0; k < P; ++k) pbar[s][k] = 0.0;
         n = a.n_acc[b] - 1;
-        load_row(n, h0, y0);
-        load_row(n - 1, h1, y1);
+#pragma unroll
+        for (int s = 0; s < 3; ++s) rows.load(n - s, hr[s], yr[s]);
         wait_vmem();
+    };
+
+    // reverse step n, whose row is in slot s, and load row n - 3 there (a lane that
+    // is done loads row 0: no branch around the load, so that the compiler's wait
+    // for it comes where it is used)
+    auto step = [&](int s) {
+        if (n >= 0) back_prop_step<Sys, Tab, Lone, NS>(tc, q, hr[s], yr[s], lam, pbar);
+        __builtin_amdgcn_sched_barrier(0);  // (the row's registers are free from here)
+        rows.load(n - 3, hr[s], yr[s]);
+        --n;
     };
 
     for (;;) {
@@ -316,7 +445,7 @@ __global__ void __launch_bounds__(256) k_rev(RevArgs a)
                 continue;
             }
             Sys::load(q, a.p, B, b, sp.kconst);
-            rows = a.traj + (size_t)b * (size_t)(sp.cap + 1) * F;
+            rows.p = a.traj + slot_rows(a.rows, a.slot ? a.slot[b] : b);
             if (a.cost) {
                 double yT[N];
 #pragma unroll
@@ -326,20 +455,27 @@ __global__ void __launch_bounds__(256) k_rev(RevArgs a)
             start_sweep();
             need = false;
         }
-        if (n >= 0) {
-            const double h = h0;
-            double y[N];
-            h0 = h1;
+        if constexpr (Lone) {
+            // a lone wave has an item per lane, so no lane waits for another's next
+            // one; three steps per trip, so that each slot keeps its registers
+            do {
+                step(0);
+                step(1);
+                step(2);
+            } while (__builtin_amdgcn_ballot_w64(n >= 0) != 0);
+        } else if (n >= 0) {
+            step(0);
+            const double h = hr[0];
+            hr[0] = hr[1];
+            hr[1] = hr[2];
+            hr[2] = h;
 #pragma unroll
             for (int i = 0; i < N; ++i) {
-                y[i] = y0[i];
-                y0[i] = y1[i];
+                const double y = yr[0][i];
+                yr[0][i] = yr[1][i];
+                yr[1][i] = yr[2][i];
+                yr[2][i] = y;
             }
-            load_row(n - 2, h1, y1);
-            // (the scheduler would move these loads to the end of the step)
-            __builtin_amdgcn_sched_barrier(0);
-            back_prop_step<Sys, Tab, Lone, NS>(tc, q, h, y, lam, pbar);
-            --n;
         }
         if (n < 0) {
 #pragma unroll
@@ -359,6 +495,98 @@ __global__ void __launch_bounds__(256) k_rev(RevArgs a)
             o += NS;
             need = o >= o_end;
             if (!need) start_sweep();
+        }
+    }
+}
+
+// The same for one seed, N = 2 and a tiled store on a full chip, by lines of four
+// rows: every fourth trip the wave keeps the lines its lanes need next in LDS and
+// loads those after them, eight lines per instruction (a lane's own loads touch a
+// line each: oscillator, B=2^20, reverse 11.6 ms, 6.0 of them vector
+// instructions).  Row r is reversed in a trip with 3 - r = trip (mod 4), so all
+// lanes need new lines at the same trip; an instance waits at most three trips for
+// its first.  Reverse 8.0 ms.
+template <class Sys, class Tab>
+__global__ void __launch_bounds__(256) k_rev_lines(RevArgs a)
+{
+    constexpr int N = Sys::N, P = Sys::P, F = N + 2;
+    static_assert(N == 2, "lines of four rows are 128 bytes for N = 2");
+    __shared__ WaveLines lines[4];
+    const int lane = threadIdx.x & 63;
+    WaveLines &wl = lines[threadIdx.x >> 6];
+    const TabRegs<Tab, false> tc;
+    const int64_t B = a.sp.B;
+    const double qnan = __builtin_nan("");
+
+    typename Sys::Params q;
+    double lam[N] = {}, pbar[P] = {};
+    int64_t b = 0;
+    int32_t n = -1;  // the next step to reverse
+    bool need = true, over = false;
+    const double *line = a.traj;  // the line with row n
+    d2 v[8];                      // lines before those in LDS, as load() gives them
+
+    for (;;) {
+        // every lane finds an instance with steps left, or none
+        bool fresh = false;
+        while (need && !over) {
+            const int64_t k = atomicAdd(a.counter, 1);
+            over = k >= B;
+            if (over) break;
+            b = a.order ? a.order[k] : k;
+            if (a.status[b] != LANE_OK) {
+#pragma unroll
+                for (int i = 0; i < N; ++i) a.lambda[(int64_t)i * B + b] = qnan;
+                for (int j = 0; j < P; ++j) a.mu[(int64_t)j * B + b] = qnan;
+                if (a.cost) a.J[b] = qnan;
+                continue;
+            }
+            Sys::load(q, a.p, B, b, a.sp.kconst);
+            if (a.cost) {
+                double yT[N];
+#pragma unroll
+                for (int i = 0; i < N; ++i) yT[i] = a.yT[(int64_t)i * B + b];
+                a.J[b] = terminal_cost<N>(a.cost, a.cost_w, yT, lam);
+            } else {
+#pragma unroll
+                for (int i = 0; i < N; ++i) lam[i] = a.lambda[(int64_t)i * B + b];
+            }
+#pragma unroll
+            for (int j = 0; j < P; ++j) pbar[j] = 0.0;
+            n = a.n_acc[b] - 1;
+            const int32_t last = n > 0 ? n : 0;
+            line = a.traj + slot_rows(a.rows, a.slot ? a.slot[b] : b) +
+                   (int64_t)(last / VA_ROW_BLOCK) * a.rows.blk;
+            need = false;
+            fresh = true;
+            wait_vmem();
+        }
+        if (__builtin_amdgcn_ballot_w64(!over) == 0) break;  // the wave, all at once
+        // a lane's first line was not loaded ahead
+        if (__builtin_amdgcn_ballot_w64(fresh) != 0) wl.load(lane, line, v);
+        wl.keep(lane, v);
+        if (n >= VA_ROW_BLOCK) line -= a.rows.blk;
+        wl.load(lane, line, v);
+        __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the steps
+#pragma unroll 1
+        for (int r = VA_ROW_BLOCK - 1; r >= 0; --r) {
+            if (n >= 0 && !over && n % VA_ROW_BLOCK == r) {
+                const double h = wl.line[lane][2 * r].y;
+                const d2 yr = wl.line[lane][2 * r + 1];
+                const double y[N] = {yr.x, yr.y};
+                back_prop_step<Sys>(tc, q, h, y, lam, pbar);
+                --n;
+            }
+        }
+        if (n < 0 && !need && !over) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) a.lambda[(int64_t)i * B + b] = lam[i];
+#pragma unroll
+            for (int j = 0; j < P; ++j) {
+                double *m = a.mu + (int64_t)j * B + b;
+                *m = a.cost || a.identity ? 0.0 + pbar[j] : *m + pbar[j];
+            }
+            need = true;
         }
     }
 }
@@ -525,6 +753,13 @@ struct Launch {
                 return hipGetLastError();
             }
         }
+        if constexpr (Sys::N == 2) {
+            if (a.slot) {
+                hipLaunchKernelGGL((k_fwd<Sys, Tab, Ad, false, true>), dim3(grid), dim3(block), 0,
+                                   s, a);
+                return hipGetLastError();
+            }
+        }
         hipLaunchKernelGGL((k_fwd<Sys, Tab, Ad, false>), dim3(grid), dim3(block), 0, s, a);
         return hipGetLastError();
     }
@@ -546,6 +781,12 @@ struct Launch {
     {
         if constexpr (Sys::N <= 4)
             if (lone_waves<Sys>(grid, block)) return rev_as<true>(a, grid, block, s);
+        if constexpr (Sys::N == 2) {
+            if (a.slot && rev_items(a).seeds == 1 && !a.identity) {
+                hipLaunchKernelGGL((k_rev_lines<Sys, Tab>), dim3(grid), dim3(block), 0, s, a);
+                return hipGetLastError();
+            }
+        }
         return rev_as<false>(a, grid, block, s);
     }
     static hipError_t pfwd(const PlainFwdArgs &a, int grid, int block, hipStream_t s)

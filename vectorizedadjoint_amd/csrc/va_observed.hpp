@@ -95,6 +95,7 @@ __global__ void __launch_bounds__(256) k_obs_fwd(ObsFwdArgs a)
     int32_t count = 0, rej = 0, tries = 0, st = LANE_OK, kobs = 0, stride = 1, nck = 0;
     bool need = true, clipped = false;
     double *row = nullptr, *ck = nullptr;  // row: row `count` of the full store
+    const int64_t row_wrap = a.st.rows.blk - (VA_ROW_BLOCK - 1) * F;
     int32_t *orow = nullptr;
 
     // The head of the controlled loop at the point (t, y): the observations
@@ -156,9 +157,9 @@ __global__ void __launch_bounds__(256) k_obs_fwd(ObsFwdArgs a)
     for (;;) {
         bool finish = false;
         if (need) {
-            b = atomicAdd(a.counter, 1);
-            if (b >= B) break;
-            if (a.order) b = a.order[b];
+            const int64_t k = atomicAdd(a.counter, 1);
+            if (k >= B) break;
+            b = a.order ? a.order[k] : k;
             Sys::load(q, a.p, B, b, sp.kconst);
 #pragma unroll
             for (int i = 0; i < N; ++i) y[i] = a.y[(int64_t)i * B + b];
@@ -184,10 +185,12 @@ __global__ void __launch_bounds__(256) k_obs_fwd(ObsFwdArgs a)
             count = rej = kobs = nck = 0;
             st = LANE_OK;
             need = false;
-            if constexpr (Ckpt)
+            if constexpr (Ckpt) {
                 ck = a.st.ck + (size_t)b * (size_t)a.st.slots * FC;
-            else
-                row = a.st.traj + (size_t)b * (size_t)(sp.cap + 1) * F;
+            } else {
+                if (a.st.slot) a.st.slot[b] = (int32_t)k;
+                row = a.st.traj + slot_rows(a.st.rows, a.st.slot ? k : b);
+            }
             orow = a.st.obs_row + (size_t)b * (size_t)K;
             tnext = obs_time(a.obs_t, K, 0, sp.t1);  // waits for the loads above as well
             if constexpr (Tab::FSAL) Sys::rhs(q, y, k0);
@@ -206,7 +209,7 @@ __global__ void __launch_bounds__(256) k_obs_fwd(ObsFwdArgs a)
                 const double tn = t + h;
                 if constexpr (!Ckpt) {
                     store_row(stored_step(tn, t));
-                    row += F;
+                    row += (count + 1) % VA_ROW_BLOCK ? F : row_wrap;
                 }
                 t = tn;
 #pragma unroll
@@ -639,32 +642,29 @@ __global__ void __launch_bounds__(256) k_obs_rev(ObsRevArgs a)
         int32_t onext = obs_point(orow, K - 1);
         int kobs = obs_jumps<N>(orow, a.obs_y, K - 1, onext, cnt, yT, lam);
         if constexpr (!Ckpt) {
-            const double *rows = a.st.traj + (size_t)b * (size_t)(sp.cap + 1) * F;
-            // rows n and n - 1, each loaded two steps before its own (as in k_rev)
-            double h0 = 0.0, h1 = 0.0, y0[N] = {}, y1[N] = {};
-            auto load_row = [&](int32_t k, double &h, double (&y)[N]) {
-                const double *r = rows + (size_t)(k > 0 ? k : 0) * F;
-                h = r[1];
+            const RowsBack<F> rows{
+                a.st.traj + slot_rows(a.st.rows, a.st.slot ? a.st.slot[b] : b),
+                (uint32_t)a.st.rows.blk * 8u};
+            // rows loaded two steps before their own, three steps per trip (as in k_rev)
+            double hr[3], yr[3][N];
+            int32_t n = cnt - 1;
 #pragma unroll
-                for (int i = 0; i < N; ++i) y[i] = r[2 + i];
-            };
-            load_row(cnt - 1, h0, y0);
-            load_row(cnt - 2, h1, y1);
+            for (int s = 0; s < 3; ++s) rows.load(n - s, hr[s], yr[s]);
             wait_vmem();
-            for (int32_t n = cnt - 1; n >= 0; --n) {
-                const double h = h0;
-                double y[N];
-                h0 = h1;
-#pragma unroll
-                for (int i = 0; i < N; ++i) {
-                    y[i] = y0[i];
-                    y0[i] = y1[i];
+            auto step = [&](int s) {
+                if (n >= 0) {
+                    back_prop_step<Sys>(tc, q, hr[s], yr[s], lam, pbar);
+                    kobs = obs_jumps<N>(orow, a.obs_y, kobs, onext, n, yr[s], lam);
                 }
-                load_row(n - 2, h1, y1);
-                __builtin_amdgcn_sched_barrier(0);  // the loads stay here
-                back_prop_step<Sys>(tc, q, h, y, lam, pbar);
-                kobs = obs_jumps<N>(orow, a.obs_y, kobs, onext, n, y, lam);
-            }
+                __builtin_amdgcn_sched_barrier(0);
+                rows.load(n - 3, hr[s], yr[s]);
+                --n;
+            };
+            do {
+                step(0);
+                step(1);
+                step(2);
+            } while (__builtin_amdgcn_ballot_w64(n >= 0) != 0);
         } else {
             const int32_t stride = a.st.stride[b];
             const double *ck = a.st.ck + (size_t)b * (size_t)a.st.slots * FC;
