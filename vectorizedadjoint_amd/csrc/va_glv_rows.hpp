@@ -262,6 +262,71 @@ __device__ __forceinline__ double adjoint_col(const double (&Acol)[NN], double w
     return ae + ao;
 }
 
+// The same for group 0 of a wave, each lane with its own u: for N <= 16 the
+// broadcast is the fused multiply-add's own (v_fmac_f64 is the one 64-bit
+// arithmetic instruction that takes a DPP row broadcast; the compiler does not fold
+// it), one instruction per term instead of two.  One statement for all terms, which
+// begins with the two wait states that a DPP read needs after u is written.
+#define VA_FMAC(k, acc, op) \
+    "v_fmac_f64_dpp %" #acc ", %2, %" #op " row_newbcast:" #k " row_mask:0xf bank_mask:0xf\n\t"
+#define VA_T1 VA_FMAC(0, 0, 3)
+#define VA_O1 "v"(A[0])
+#define VA_T2 VA_T1 VA_FMAC(1, 1, 4)
+#define VA_O2 VA_O1, "v"(A[1])
+#define VA_T3 VA_T2 VA_FMAC(2, 0, 5)
+#define VA_O3 VA_O2, "v"(A[2])
+#define VA_T4 VA_T3 VA_FMAC(3, 1, 6)
+#define VA_O4 VA_O3, "v"(A[3])
+#define VA_T5 VA_T4 VA_FMAC(4, 0, 7)
+#define VA_O5 VA_O4, "v"(A[4])
+#define VA_T6 VA_T5 VA_FMAC(5, 1, 8)
+#define VA_O6 VA_O5, "v"(A[5])
+#define VA_T7 VA_T6 VA_FMAC(6, 0, 9)
+#define VA_O7 VA_O6, "v"(A[6])
+#define VA_T8 VA_T7 VA_FMAC(7, 1, 10)
+#define VA_O8 VA_O7, "v"(A[7])
+#define VA_T9 VA_T8 VA_FMAC(8, 0, 11)
+#define VA_O9 VA_O8, "v"(A[8])
+#define VA_T10 VA_T9 VA_FMAC(9, 1, 12)
+#define VA_O10 VA_O9, "v"(A[9])
+#define VA_T11 VA_T10 VA_FMAC(10, 0, 13)
+#define VA_O11 VA_O10, "v"(A[10])
+#define VA_T12 VA_T11 VA_FMAC(11, 1, 14)
+#define VA_O12 VA_O11, "v"(A[11])
+#define VA_T13 VA_T12 VA_FMAC(12, 0, 15)
+#define VA_O13 VA_O12, "v"(A[12])
+#define VA_T14 VA_T13 VA_FMAC(13, 1, 16)
+#define VA_O14 VA_O13, "v"(A[13])
+#define VA_T15 VA_T14 VA_FMAC(14, 0, 17)
+#define VA_O15 VA_O14, "v"(A[14])
+#define VA_T16 VA_T15 VA_FMAC(15, 1, 18)
+#define VA_O16 VA_O15, "v"(A[15])
+#define VA_TERMS(n)                                                    \
+    if constexpr (NN == n)                                             \
+        asm("s_nop 1\n\t" VA_T##n : "+&v"(ae), "+&v"(ao) : "v"(u), VA_O##n)
+template <int NN>
+__device__ __forceinline__ void adjoint_terms(const double (&A)[NN], double u, double &ae,
+                                              double &ao)
+{
+    VA_TERMS(2); VA_TERMS(3); VA_TERMS(4); VA_TERMS(5); VA_TERMS(6);
+    VA_TERMS(7); VA_TERMS(8); VA_TERMS(9); VA_TERMS(10); VA_TERMS(11);
+    VA_TERMS(12); VA_TERMS(13); VA_TERMS(14); VA_TERMS(15); VA_TERMS(16);
+}
+#undef VA_TERMS
+template <int NN>
+__device__ __forceinline__ double adjoint_col_group0(const double (&Acol)[NN], double wg, double u)
+{
+    if constexpr (NN <= 16) {
+        double ae = wg, ao = 0.0;
+        adjoint_terms<NN>(Acol, u, ae, ao);
+        return ae + ao;
+    } else {
+        double vu[NN];
+        bcast_group0<NN>(u, vu);
+        return adjoint_col<NN>(Acol, wg, vu);
+    }
+}
+
 // Where a group's instances come from: the persistent kernels take queue
 // positions [lo, hi) from an atomic counter (mapped through `order` when given;
 // `split`/`part` select the positions below or from *split); OneShot bodies
@@ -995,12 +1060,17 @@ __device__ __forceinline__ bool wait_above(Ring &R, int *ctr, int k)
     return false;
 }
 
-// Wave 1: stage values of steps n_acc-1 .. 0 into the ring.
+// Wave 1: stage values of steps n_acc-1 .. 0 into the ring, R steps per pass, one
+// in each 16-lane row (N <= 16): the steps do not depend on one another, and one
+// at a time wave 1 was slower than wave 0's recursion (254 instructions a step).
 template <int NN, class Tab, bool IM>
 __device__ __forceinline__ void glv_long_stage(const RevArgs &a, int64_t b, StageRing<NN, Tab> &R)
 {
     constexpr int S = Tab::S, F = NN + 2;
-    const int i = threadIdx.x & 63;
+    constexpr int ROWS = NN <= 16 ? 4 : 1;
+    static_assert(VA_STAGE_RING >= 2 * ROWS, "a pass is staged while another is reversed");
+    const int lane = threadIdx.x & 63;
+    const int i = ROWS > 1 ? lane & 15 : lane, row = ROWS > 1 ? lane >> 4 : 0;
     if (i >= NN) return;
     __builtin_amdgcn_s_setprio(3);
     const SolveParams sp = a.sp;
@@ -1013,25 +1083,22 @@ __device__ __forceinline__ void glv_long_stage(const RevArgs &a, int64_t b, Stag
     for (int j = 0; j < NN; ++j) Arow[j] = param<NN, IM>(a, NN * (i + 1) + j, b);
     const double *rows = a.traj + (size_t)b * (size_t)(sp.cap + 1) * F;
     const TabRegs<Tab, true> tc;
-    // (h_n, y_n,i) of the next two steps, loaded ahead of use
-    int n = nacc - 1;
-    double h0 = rows[(size_t)n * F + 1], y0 = rows[(size_t)n * F + 2 + i], h1 = 0.0, y1 = 0.0;
-    if (n >= 1) {
-        h1 = rows[(size_t)(n - 1) * F + 1];
-        y1 = rows[(size_t)(n - 1) * F + 2 + i];
-    }
-    for (int k = 0; k < nacc; ++k, --n) {
+    // (h_n, y_n,i) of this row's step of the next two passes, loaded ahead of use
+    // (row 0 of the trajectory below the first)
+    int n = nacc - 1 - row;
+    auto at = [&](int m) { return rows + (size_t)(m > 0 ? m : 0) * F; };
+    double h0 = at(n)[1], y0 = at(n)[2 + i];
+    double h1 = at(n - ROWS)[1], y1 = at(n - ROWS)[2 + i];
+    for (int k = 0; k < nacc; k += ROWS, n -= ROWS) {
         const double h = h0, y = y0;
         h0 = h1;
         y0 = y1;
-        if (n >= 2) {
-            h1 = rows[(size_t)(n - 2) * F + 1];
-            y1 = rows[(size_t)(n - 2) * F + 2 + i];
-        }
-        // the slot of step k - RING must have been accumulated by wave 2 (and so
-        // read by wave 0 before that)
-        if (k >= VA_STAGE_RING && !wait_above(R, &R.done, k - VA_STAGE_RING)) return;
-        const int slot = k % VA_STAGE_RING;
+        h1 = at(n - 2 * ROWS)[1];
+        y1 = at(n - 2 * ROWS)[2 + i];
+        // the slots of the steps VA_STAGE_RING before must have been accumulated by
+        // wave 2 (and so read by wave 0 before that)
+        if (k + ROWS > VA_STAGE_RING && !wait_above(R, &R.done, k + ROWS - 1 - VA_STAGE_RING)) return;
+        const int slot = (k + row) % VA_STAGE_RING;
         double Kn[S];
 #pragma unroll
         for (int m = 0; m < S; ++m) {
@@ -1045,9 +1112,9 @@ __device__ __forceinline__ void glv_long_stage(const RevArgs &a, int64_t b, Stag
             R.xg[slot][m][i] = make_double2(x, g);
         }
         R.h[slot] = h;
-        // the slot's writes complete before the count that publishes them
+        // the slots' writes complete before the count that publishes them
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        ring_store(&R.avail, k + 1);
+        ring_store(&R.avail, k + ROWS < nacc ? k + ROWS : nacc);
     }
 }
 
@@ -1072,7 +1139,7 @@ __device__ __forceinline__ void glv_long_backward(const RevArgs &a, int64_t b,
         return;
     }
     const TabRegs<Tab, true> tc;
-    double Acol[NN], v[NN], vu[NN], lam;
+    double Acol[NN], v[NN], lam;
 #pragma unroll
     for (int j = 0; j < NN; ++j) Acol[j] = param<NN, IM>(a, NN * (j + 1) + i, b);
     if (a.cost) {
@@ -1094,93 +1161,116 @@ __device__ __forceinline__ void glv_long_backward(const RevArgs &a, int64_t b,
         lam = a.lambda[(int64_t)i * B + b];
     }
     const int32_t nacc = a.n_acc[b];
-    for (int k = 0; k < nacc; ++k) {
-        if (!wait_above(R, &R.avail, k)) {
-            lam = qnan;
-            break;
-        }
+    // The values of step k + 1 are read into the registers that step k has done
+    // with, so the recursion does not wait for LDS; where wave 1 had not staged
+    // them yet they are read again.
+    double X[S], G[S], h = 0.0;
+    auto read_stage = [&](int slot, int m) {
+        const double2 xg = R.xg[slot][m][i];
+        X[m] = xg.x;
+        G[m] = xg.y;
+    };
+    int avail = 0;  // steps known to be staged
+    // step k's values, once staged; false when the wait gives up
+    auto read_step = [&](int k) {
+        if (!wait_above(R, &R.avail, k)) return false;
+        avail = k + 1;
         const int slot = k % VA_STAGE_RING;
-        double X[S], G[S];
 #pragma unroll
-        for (int m = 0; m < S; ++m) {
-            const double2 xg = R.xg[slot][m][i];
-            X[m] = xg.x;
-            G[m] = xg.y;
+        for (int m = 0; m < S; ++m) read_stage(slot, m);
+        h = R.h[slot];
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): none left for the loop to wait for
+        return true;
+    };
+    bool ok = nacc <= 0 || read_step(0);
+    for (int k = 0; ok && k < nacc;) {
+        const int slot = k % VA_STAGE_RING, next = (k + 1) % VA_STAGE_RING;
+        if (avail <= k + 1) {
+            avail = __builtin_amdgcn_readfirstlane(ring_load(&R.avail));
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
         }
-        const double h = R.h[slot];
         double Kb[S];
+        const double hk = h;
+        h = R.h[next];
 #pragma unroll
-        for (int m = 0; m < S; ++m) Kb[m] = (tc.b[m] * h) * lam;
+        for (int m = 0; m < S; ++m) Kb[m] = (tc.b[m] * hk) * lam;
         double ybar = lam;
 #pragma unroll
         for (int ii = 0; ii < S; ++ii) {
             const int m = S - 1 - ii;
             const double w = Kb[m];
-            const double xown = X[m];
-            const double u = w * xown;
+            const double u = w * X[m];
             const double wg = w * G[m];
+            __builtin_amdgcn_sched_barrier(0);  // (X[m] and G[m] are free from here)
+            read_stage(next, m);
             R.u[slot][m][i] = u;
-            bcast_group0<NN>(u, vu);
-            const double xi = adjoint_col<NN>(Acol, wg, vu);
+            const double xi = adjoint_col_group0<NN>(Acol, wg, u);
             ybar = ybar + xi;
             // Kbar_j += (xi a_mj) h (detail/backpropagation.hpp:215)
 #pragma unroll
             for (int j = 0; j < S; ++j)
-                if (j < m && Tab::A[m][j] != 0.0) Kb[j] = Kb[j] + (xi * tc.a[m][j]) * h;
+                if (j < m && Tab::A[m][j] != 0.0) Kb[j] = Kb[j] + (xi * tc.a[m][j]) * hk;
         }
         lam = ybar;
         // the step's products are written before the count that publishes them
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        ring_store(&R.uavail, k + 1);
+        ring_store(&R.uavail, ++k);
+        if (avail <= k && k < nacc) ok = read_step(k);
     }
+    if (!ok) lam = qnan;
     a.lambda[(int64_t)i * B + b] = lam;
 }
 
 // Wave 2: dJ/dr_i and column i of dJ/dA from the products u of each step wave 0
 // has reversed, in wave 0's stage order (what glv_rows_rev_body accumulates
-// beside its recursion, the same operations in the same order).
+// beside its recursion, the same operations in the same order).  The wave's 64/N
+// groups of lanes share a column's entries, E each: with all of them in one lane
+// wave 2 was slower than wave 0's recursion (256 instructions a step).
 template <int NN, class Tab, bool IM>
 __device__ __forceinline__ void glv_long_accumulate(const RevArgs &a, int64_t b,
                                                     StageRing<NN, Tab> &R)
 {
-    constexpr int S = Tab::S;
-    const int i = threadIdx.x & 63;
-    if (i >= NN) return;
+    constexpr int S = Tab::S, GPW = 64 / NN, E = (NN + GPW - 1) / GPW;
+    const int lane = threadIdx.x & 63;
+    const int grp = lane / NN, i = lane - grp * NN;
+    if (grp * E >= NN) return;
     __builtin_amdgcn_s_setprio(3);
     // wave 0 writes the outputs of an instance that did not end OK
     if (a.status[b] != LANE_OK) return;
     const double qnan = __builtin_nan("");
-    double Abar[NN], vu[NN], rbar = 0.0;
+    double Abar[E], rbar = 0.0;
+    int row[E];  // entries (row, i) of dJ/dA; past the last one that one once more
 #pragma unroll
-    for (int j = 0; j < NN; ++j) Abar[j] = 0.0;
+    for (int e = 0; e < E; ++e) {
+        Abar[e] = 0.0;
+        row[e] = grp * E + e < NN ? grp * E + e : NN - 1;
+    }
     const int32_t nacc = a.n_acc[b];
     for (int k = 0; k < nacc; ++k) {
         if (!wait_above(R, &R.uavail, k)) {
             rbar = qnan;
 #pragma unroll
-            for (int j = 0; j < NN; ++j) Abar[j] = qnan;
+            for (int e = 0; e < E; ++e) Abar[e] = qnan;
             break;
         }
         const int slot = k % VA_STAGE_RING;
 #pragma unroll
         for (int ii = 0; ii < S; ++ii) {
             const int m = S - 1 - ii;
-#pragma unroll
-            for (int kk = 0; kk < NN; ++kk) vu[kk] = R.u[slot][m][kk];
             const double xown = R.xg[slot][m][i].x;
-            const double u = R.u[slot][m][i];
-            rbar = rbar + u;
-            // column i of dJ/dA: dA_ki += u_k X_i, each product rounded before it is added
+            rbar = rbar + R.u[slot][m][i];
+            // dA_ki += u_k X_i, each product rounded before it is added
 #pragma unroll
-            for (int kk = 0; kk < NN; ++kk) Abar[kk] = Abar[kk] + vu[kk] * xown;
+            for (int e = 0; e < E; ++e) Abar[e] = Abar[e] + R.u[slot][m][row[e]] * xown;
         }
         // the slot's values are read: release it to waves 0 and 1
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         ring_store(&R.done, k + 1);
     }
-    put_pbar<NN, IM>(a, 0, i, b, rbar);
+    if (grp == 0) put_pbar<NN, IM>(a, 0, i, b, rbar);
 #pragma unroll
-    for (int kk = 0; kk < NN; ++kk) put_pbar<NN, IM>(a, 0, NN * (kk + 1) + i, b, Abar[kk]);
+    for (int e = 0; e < E; ++e)
+        if (grp * E + e < NN) put_pbar<NN, IM>(a, 0, NN * (row[e] + 1) + i, b, Abar[e]);
 }
 
 // The persistent reverse.  With part 2 (one seed) the head of the order, instances
