@@ -256,6 +256,7 @@ struct OrderArgs {
     const int32_t *from;  // the scatter takes instances in this order (null: index order)
     int32_t *work;   // per mode a histogram and cursors, cleared before
     int32_t *order[2], *n_long[2];
+    int long_bucket[2];
 };
 
 __global__ void __launch_bounds__(VA_ORDER_BUCKETS) k_order_hist(OrderArgs a, CountsOut out)
@@ -280,9 +281,16 @@ __global__ void __launch_bounds__(VA_ORDER_BUCKETS) k_order_hist(OrderArgs a, Co
             atomicAdd(&a.work[2 * m * VA_ORDER_BUCKETS + threadIdx.x], cnt[m][threadIdx.x]);
 }
 
-// The instances in buckets >= VA_LONG_BUCKET, at most VA_LONG_MAX, are the head of
-// an order that the long-instance kernels take; their count goes to n_long.
-constexpr int VA_LONG_BUCKET = 32;  // 256 attempts (or accepted steps) and more
+// The instances in buckets >= OrderArgs::long_bucket, at most VA_LONG_MAX, are the
+// head of an order that the long-instance kernels take; their count goes to n_long.
+// For a forward that is 256 attempts and more, or, with a batch above 5/3 of the
+// lanes in flight, 448: the bulk beside the long instances then ends last, and the
+// long kernel's waves, one instance each, take more from it than the instances
+// do (GLV, t1=50, solve at 256 / 448: N=10, lanes 36864, B=48000 1.88 / 1.99 ms,
+// 58000 2.12 / 2.12, 65536 2.38 / 2.29, 80000 2.95 / 2.84; N=5, lanes 73728,
+// B=150000 4.47 / 4.38; N=16, lanes 24576, B=40000 5.44 / 5.50).
+constexpr int VA_LONG_BUCKET = 32;       // 256 attempts (or accepted steps)
+constexpr int VA_LONG_BUCKET_FULL = 56;  // 448
 constexpr int VA_LONG_MAX = 256;    // one block each
 constexpr int VA_REV_LONG = 4;      // where in va_handle::counters a reverse order's count lies
 
@@ -306,7 +314,7 @@ __global__ void __launch_bounds__(VA_ORDER_BUCKETS) k_order_scatter(OrderArgs a)
             sfx[k] += v;
             __syncthreads();
         }
-        if (blockIdx.x == 0 && k == VA_LONG_BUCKET)
+        if (blockIdx.x == 0 && k == a.long_bucket[m])
             *a.n_long[m] = sfx[k] < VA_LONG_MAX ? sfx[k] : VA_LONG_MAX;
         int bucket[VA_ORDER_ITEMS], rank[VA_ORDER_ITEMS], inst[VA_ORDER_ITEMS];
 #pragma unroll
@@ -576,6 +584,8 @@ va_status build_orders(va_handle *h, int modes, bool next, const CountsOut &out,
     a.n_long[0] = h->counters + VA_REV_LONG;
     a.order[1] = next ? h->order_fwd_next : h->order_fwd;
     a.n_long[1] = h->counters + (next ? 11 - h->nlong_idx : h->nlong_idx);
+    a.long_bucket[0] = VA_LONG_BUCKET;
+    a.long_bucket[1] = 3 * a.B > 5 * h->lanes_fwd ? VA_LONG_BUCKET_FULL : VA_LONG_BUCKET;
     if (modes & 2) h->ordered = true;
     const int grid = blocks_for(a.B, VA_ORDER_BUCKETS * a.items);
     hipLaunchKernelGGL(k_order_hist, dim3(grid), dim3(VA_ORDER_BUCKETS), 0, s, a, out);
