@@ -1166,10 +1166,10 @@ TuneKey tune_key(const va_problem *pb, int device)
     return TuneKey{device, pb->system, pb->n_state, pb->tableau, pb->adaptive, pb->n_obs, bucket};
 }
 
-// Instances from which a one-lane store is tiled: below, the rows of a few waves are
-// in reach of the translation caches however they lie, and a lone wave's reverse
-// was slower on tiles (Van der Pol, B=1024: reverse 0.78 ms instance-major, 0.86
-// tiled; RK4 oscillator, B=40000: solve 1.16 ms instance-major, 1.04 tiled).
+// Instances from which a one-lane store is tiled: the rows of a few waves are in reach
+// of the translation caches however they lie (Van der Pol, B=1024: forward 1.05 ms,
+// reverse 0.69 ms either way), where the tiles' padding would be large against the
+// batch; RK4 oscillator, B=40000: solve 1.16 ms instance-major, 1.04 tiled.
 constexpr int64_t VA_TILED_MIN = 4096;
 
 va_status create_handle(const va_problem *pb_in, const va::KernelSet *given, va_handle **out)
@@ -1358,10 +1358,23 @@ va_status create_handle(const va_problem *pb_in, const va::KernelSet *given, va_
             // one-lane kernels that know tiled rows have them in large stores, the
             // others instance-major
             const int F = ks.n + 2;
-            if (ks.layout == 0 && ks.table_version >= 2 && B >= VA_TILED_MIN) {
+            bool tiled = ks.layout == 0 && ks.table_version >= 2 && B >= VA_TILED_MIN;
+            if (tiled && e == hipSuccess) {
+                // whole tiles and blocks of rows take more than the rows: instance-major
+                // where only that fits the budget or the device
                 h->rows = va::rows_tiled(pb->max_steps, F);
                 const size_t tiles = ((size_t)B + va::VA_ROW_TILE - 1) / va::VA_ROW_TILE;
-                alloc((void **)&h->traj, sizeof(double) * tiles * (size_t)h->rows.tile);
+                const size_t bytes = sizeof(double) * tiles * (size_t)h->rows.tile;
+                if (budget > 0.0 &&
+                    (double)bytes + 4.0 * (double)B * ((double)pb->n_obs + 1.0) > budget) {
+                    tiled = false;
+                } else if (hipMalloc((void **)&h->traj, bytes) != hipSuccess) {
+                    (void)hipGetLastError();
+                    h->traj = nullptr;
+                    tiled = false;
+                }
+            }
+            if (tiled) {
                 alloc((void **)&h->slot, sizeof(int32_t) * (size_t)B);
             } else {
                 h->rows = va::rows_instance_major(pb->max_steps, F);
