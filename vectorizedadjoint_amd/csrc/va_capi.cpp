@@ -104,6 +104,13 @@ __global__ void k_copy_counts(CountsOut out, const int32_t *s_acc, const int32_t
     if (out.status) out.status[i] = s_st[i];
 }
 
+// n_acc[i] at most `most`.
+__global__ void k_cap_counts(int32_t *n_acc, int64_t n, int32_t most)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n && n_acc[i] > most) n_acc[i] = most;
+}
+
 __global__ void k_identity_seeds(double *lambda, int n, int64_t B)
 {
     // lambda[o][i][b] = (o == i)
@@ -1258,8 +1265,7 @@ va_status create_handle(const va_problem *pb_in, const va::KernelSet *given, va_
             const int64_t rev_threads =
                 (int64_t)blocks_for(std::min<int64_t>(h->lanes_obs_rev, B), h->block) * h->block;
             auto cost = [&](int32_t slots, int32_t *stride_max) {
-                int32_t sm = 1;
-                while ((int64_t)sm * slots < (int64_t)pb->max_steps) sm *= 2;
+                const int32_t sm = va::obs_stride_max(pb->max_steps, slots);
                 *stride_max = sm;
                 return 8.0 * (double)B * slots * (ks.n + 3) +
                        8.0 * (double)rev_threads * sm * (ks.n + 1) + fixed;
@@ -1269,8 +1275,7 @@ va_status create_handle(const va_problem *pb_in, const va::KernelSet *given, va_
             // ceil(stride_max / slots2) rows
             auto cost2 = [&](int32_t slots, int32_t *stride_max, int32_t *slots2,
                              int32_t *seg_rows) {
-                int32_t sm = 1;
-                while ((int64_t)sm * slots < (int64_t)pb->max_steps) sm *= 2;
+                const int32_t sm = va::obs_stride_max(pb->max_steps, slots);
                 int32_t s2 = 2;
                 while ((int64_t)s2 * s2 < sm) s2 *= 2;
                 *stride_max = sm;
@@ -1685,6 +1690,13 @@ static va_status observed_enqueue(va_handle *h, const double *y0, const double *
     f.K = h->pb.n_obs;
     f.J = J;
     f.st = os;
+    if (h->obs_ckpt && h->pb.system == VA_SYSTEM_USER) {
+        // kernels that a caller built before obs_first_stride() start from twice
+        // stride_max after an instance that took all of its steps
+        hipLaunchKernelGGL(k_cap_counts, dim3(blocks_for(B, 256)), dim3(256), 0, s, h->n_acc, B,
+                           h->pb.max_steps - 1);
+        VA_HIP(hipGetLastError());
+    }
     VA_HIP(h->ks.obs_fwd(f, blocks_for(std::min<int64_t>(h->lanes_obs_fwd, B), h->block),
                          h->block, s));
     h->have_forward = !h->obs_ckpt;

@@ -162,6 +162,29 @@ struct ObsStore {
     int32_t *slot = nullptr;
 };
 
+// The largest checkpoint spacing a solve of at most cap steps can need with `slots`
+// checkpoints: the row buffers of the reverse are sized for it.  Spacings are
+// powers of two; doubled only where a checkpoint is due and no slot is free, which
+// with this one does not happen (slots * it >= cap, checkpoints lie below cap).
+__host__ __device__ inline int32_t obs_stride_max(int64_t cap, int32_t slots)
+{
+    int32_t s = 1;
+    while ((int64_t)s * slots < cap) s *= 2;
+    return s;
+}
+
+// The spacing a solve starts from after one of `prev` accepted steps: the smallest
+// with room for that many and never above stride_max, which the row buffers of
+// the reverse are sized for (prev may be the cap itself, after an instance that
+// ran out of steps).
+__host__ __device__ inline int32_t obs_first_stride(int32_t prev, int32_t slots,
+                                                    int32_t stride_max)
+{
+    int32_t s = 1;
+    while (s < stride_max && (int64_t)s * slots <= prev) s *= 2;
+    return s;
+}
+
 struct ObsFwdArgs {
     SolveParams sp;
     double *y;             // [N][B] in y0, out y(T)

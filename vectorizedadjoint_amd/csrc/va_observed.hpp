@@ -177,10 +177,7 @@ __global__ void __launch_bounds__(256) k_obs_fwd(ObsFwdArgs a)
                 // that spacing, which filled the slots once per solve, cost 10% of
                 // the observed Van der Pol solve).  Any spacing gives the same
                 // results: the reverse replays the forward from each checkpoint.
-                if (a.order) {
-                    const int32_t prev = a.n_acc[b];
-                    while ((int64_t)stride * a.st.slots <= prev) stride *= 2;
-                }
+                if (a.order) stride = obs_first_stride(a.n_acc[b], a.st.slots, a.st.stride_max);
             }
             count = rej = kobs = nck = 0;
             st = LANE_OK;
