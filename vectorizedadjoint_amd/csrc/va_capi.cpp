@@ -255,18 +255,7 @@ __device__ __forceinline__ int order_bucket(const int32_t *n_acc, const int32_t 
     return k < VA_ORDER_BUCKETS - 1 ? k : VA_ORDER_BUCKETS - 1;
 }
 
-struct OrderArgs {
-    const int32_t *n_acc, *n_rej, *status;
-    int64_t B;
-    int modes;       // bit 0: the reverse order, bit 1: the forward order
-    int items;       // instances per thread, at most VA_ORDER_ITEMS
-    const int32_t *from;  // the scatter takes instances in this order (null: index order)
-    int32_t *work;   // per mode a histogram and cursors, cleared before
-    int32_t *order[2], *n_long[2];
-    int long_bucket[2];
-};
-
-__global__ void __launch_bounds__(VA_ORDER_BUCKETS) k_order_hist(OrderArgs a, CountsOut out)
+__global__ void __launch_bounds__(VA_ORDER_BUCKETS) k_order_hist(va::OrderArgs a, CountsOut out)
 {
     __shared__ int32_t cnt[2][VA_ORDER_BUCKETS];
     cnt[0][threadIdx.x] = cnt[1][threadIdx.x] = 0;
@@ -288,7 +277,7 @@ __global__ void __launch_bounds__(VA_ORDER_BUCKETS) k_order_hist(OrderArgs a, Co
             atomicAdd(&a.work[2 * m * VA_ORDER_BUCKETS + threadIdx.x], cnt[m][threadIdx.x]);
 }
 
-// The instances in buckets >= OrderArgs::long_bucket, at most VA_LONG_MAX, are the
+// The instances in buckets >= va::OrderArgs::long_bucket, at most VA_LONG_MAX, are the
 // head of an order that the long-instance kernels take; their count goes to n_long.
 // For a forward that is 256 attempts and more, or, with a batch above 5/3 of the
 // lanes in flight, 448: the bulk beside the long instances then ends last, and the
@@ -301,7 +290,7 @@ constexpr int VA_LONG_BUCKET_FULL = 56;  // 448
 constexpr int VA_LONG_MAX = 256;    // one block each
 constexpr int VA_REV_LONG = 4;      // where in va_handle::counters a reverse order's count lies
 
-__global__ void __launch_bounds__(VA_ORDER_BUCKETS) k_order_scatter(OrderArgs a)
+__global__ void __launch_bounds__(VA_ORDER_BUCKETS) k_order_scatter(va::OrderArgs a)
 {
     __shared__ int32_t sfx[VA_ORDER_BUCKETS], cnt[VA_ORDER_BUCKETS];
     const int k = threadIdx.x;
@@ -465,7 +454,6 @@ struct va_handle {
     // and the end of the bulk's forward)
     hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_fwd = nullptr;
-    bool capturing = false;  // solve_enqueue is being recorded into a graph
 };
 
 namespace {
@@ -578,7 +566,7 @@ va_status clear_and_copy(va_handle *h, double *yT, const double *y0, hipStream_t
 va_status build_orders(va_handle *h, int modes, bool next, const CountsOut &out, hipStream_t s,
                        const int32_t *from = nullptr)
 {
-    OrderArgs a;
+    va::OrderArgs a;
     a.n_acc = h->n_acc;
     a.n_rej = h->n_rej;
     a.status = h->status;
@@ -601,6 +589,20 @@ va_status build_orders(va_handle *h, int modes, bool next, const CountsOut &out,
     return VA_OK;
 }
 
+// Whether what goes to s is recorded into a graph, the library's own or the
+// caller's: a recording runs later and again, so no buffers are swapped for it (its
+// replays would not read the order that the one before left, and a call before the
+// first replay would read the one that is not written yet).
+bool recording(hipStream_t s)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
 // The orders after a forward of the one-lane kernels that took instances in the
 // order `taken`: neighbours of that order, whose rows are neighbours, stay
 // together in the reverse's.  A recorded solve, whose replays share one buffer,
@@ -608,7 +610,7 @@ va_status build_orders(va_handle *h, int modes, bool next, const CountsOut &out,
 va_status orders_after(va_handle *h, int modes, const int32_t *taken, const CountsOut &out,
                        hipStream_t s)
 {
-    if (h->capturing || !taken) return build_orders(h, modes, false, out, s);
+    if (!taken || recording(s)) return build_orders(h, modes, false, out, s);
     if (va_status st = build_orders(h, modes, true, out, s, taken)) return st;
     if (modes & 2) {
         std::swap(h->order_fwd, h->order_fwd_next);
@@ -952,7 +954,7 @@ va_status solve_split(va_handle *h, const double *y0, double *yT, const double *
     // the order into the spare buffer.  A solve recorded into a graph builds it
     // after the join into the same buffer, so that every replay reads the order
     // the previous replay left.
-    const bool ahead = !h->capturing;
+    const bool ahead = !recording(s);
     if (ahead) {
         VA_HIP(hipEventRecord(h->ev_fwd, h->side));
         VA_HIP(hipStreamWaitEvent(s, h->ev_fwd, 0));
@@ -1423,10 +1425,12 @@ va_status create_handle(const va_problem *pb_in, const va::KernelSet *given, va_
     if (e == hipSuccess) e = hipMemset(h->counters, 0, sizeof(int32_t) * VA_WORK_INTS);
     if (e == hipSuccess) e = hipMemset(h->n_acc, 0, sizeof(int32_t) * B);
     if (e == hipSuccess) e = hipMemset(h->n_rej, 0, sizeof(int32_t) * B);
-    {  // the first forward takes instances in index order
-        if (e == hipSuccess) {
-            hipLaunchKernelGGL(k_iota_i32, dim3(blocks_for(B, 256)), dim3(256), 0, nullptr,
-                               h->order_fwd, B);
+    {  // the first forward takes instances in index order; every order (and slot) names
+        // instances from here on, whatever a recorded and not yet run solve leaves out
+        for (int32_t *order : {h->order_fwd, h->order_fwd_next, h->order, h->slot}) {
+            if (e != hipSuccess || !order) continue;
+            hipLaunchKernelGGL(k_iota_i32, dim3(blocks_for(B, 256)), dim3(256), 0, nullptr, order,
+                               B);
             e = hipGetLastError();
         }
         if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
@@ -1582,10 +1586,8 @@ va_status va_solve(va_handle *h, const double *y0, const double *p, int32_t cost
             h->graph_exec = nullptr;
         }
         VA_HIP(hipStreamBeginCapture(h->cap_stream, hipStreamCaptureModeThreadLocal));
-        h->capturing = true;
         st = solve_enqueue(h, y0, p, cost, cost_weights, J, yT, dJdy0, dJdp, n_accepted,
                            n_rejected, lane_status, h->cap_stream);
-        h->capturing = false;
         hipGraph_t graph = nullptr;
         const hipError_t ec = hipStreamEndCapture(h->cap_stream, &graph);
         if (st) {

@@ -285,6 +285,18 @@ struct KernelSet {
     int shared_waves;            // waves per workgroup of the shared-parameter kernels
 };
 
+// The kernels that order instances longest first (va_capi.cpp).
+struct OrderArgs {
+    const int32_t *n_acc, *n_rej, *status;
+    int64_t B;
+    int modes;       // bit 0: the reverse order, bit 1: the forward order
+    int items;       // instances per thread, at most VA_ORDER_ITEMS (va_capi.cpp)
+    const int32_t *from;  // the scatter takes instances in this order (null: index order)
+    int32_t *work;   // per mode a histogram and cursors, cleared before
+    int32_t *order[2], *n_long[2];
+    int long_bucket[2];
+};
+
 hipError_t launch_glvs_reduce(const double *part, int nparts, double *out, hipStream_t s);
 
 // Returns false when (system, n, tableau, adaptive) has no compiled kernels.
