@@ -72,7 +72,7 @@ void log_launch(const void *f, dim3 g, dim3 b, void **args)
     free(d);
     for (const char *drop : {"void ", "va::", "(anonymous namespace)::"})
         for (size_t k; (k = n.find(drop)) != std::string::npos;) n.erase(k, strlen(drop));
-    n = n.substr(0, n.find('('));
+    n = n.substr(0, n.rfind('('));
     while (!n.empty() && n.back() == ' ') n.pop_back();
     if (starts(n, "k_iota_i32") && !capturing) written.insert(*(void **)args[0]);
     if (starts(n, "k_order_scatter") && !capturing) {

@@ -252,7 +252,7 @@ __global__ void __launch_bounds__(256) k_fwd(FwdArgs a)
         if constexpr (Lines)
             if (__builtin_amdgcn_ballot_w64(!over) == 0) break;  // the wave, all at once
         if constexpr (Lone) {
-            // (a lone wave has an instance per lane: no lane waits for another's refill)
+            // (no refill until all of the wave's lanes are done: see VA_LONE_THREADS)
             while (!finish) attempt(finish, full);
         } else if (!finish && !over) {
             attempt(finish, full);
@@ -456,8 +456,8 @@ __global__ void __launch_bounds__(256) k_rev(RevArgs a)
             need = false;
         }
         if constexpr (Lone) {
-            // a lone wave has an item per lane, so no lane waits for another's next
-            // one; three steps per trip, so that each slot keeps its registers
+            // three steps per trip, so that each slot keeps its registers; no refill
+            // until all of the wave's lanes are done (see VA_LONE_THREADS)
             do {
                 step(0);
                 step(1);
@@ -733,22 +733,65 @@ __global__ void __launch_bounds__(256) k_plain_rev(PlainRevArgs a)
 // ---------------------------------------------------------------------------
 // A launch whose waves have a SIMD each (at most one wave per SIMD of the 256
 // CUs): its time is the waves' own instruction count, and it takes the kernels
-// with the constants in vector registers.  Only small systems have them: the
-// state of a larger one needs the registers.
+// with the constants in vector registers (Lone).  With more instances than lanes
+// as well, where a wave takes new ones only when all of its own have ended: Van
+// der Pol, B=131072 on 4096 lanes, forward 10.2 ms against 16.1 of the refilling
+// kernel, in index order 16.5 / 17.6; Lotka-Volterra N=4, one lane each, on
+// 16384 lanes 0.49 / 0.97 and 0.61 / 1.41.
 constexpr int VA_LONE_THREADS = 256 * 4 * 64;
+inline bool lone_waves(int grid, int block) { return (int64_t)grid * block <= VA_LONE_THREADS; }
 
-template <class Sys>
-inline bool lone_waves(int grid, int block)
+// Only sweeps whose values fit beside the constants have such kernels: a lane has
+// 512 registers, 256 doubles, and the compiler needs some third of them for
+// intermediates.  Reverses with one seed, B=65536, Lone against not, by the doubles
+// counted here: Lotka-Volterra N=4, Cash-Karp (107) 332 / 430 us; N=2, Fehlberg
+// 7(8) (126) 129 / 131; N=3, Fehlberg (164) 185 / 241; N=4, Fehlberg (206, which
+// puts 592 bytes per lane in scratch memory) 810 / 641 us.
+constexpr int VA_LONE_DOUBLES = 168;
+
+constexpr int count_nonzero(const double *v, int n)
 {
-    return Sys::N <= 4 && (int64_t)grid * block <= VA_LONE_THREADS;
+    int c = 0;
+    for (int k = 0; k < n; ++k) c += v[k] != 0.0;
+    return c;
+}
+// the stage weights of the first `stages` stages, and the solution's
+template <class Tab>
+constexpr int stage_constants(int stages)
+{
+    int c = count_nonzero(Tab::B, Tab::S);
+    for (int m = 1; m < stages; ++m) c += count_nonzero(Tab::A[m], m);
+    return c;
+}
+// the embedded error's weights and the controller's pow (PowRegs)
+template <class Tab>
+constexpr int control_constants()
+{
+    if constexpr (Tab::HAS_ERR) return count_nonzero(Tab::DB, Tab::SF) + 17;
+    else return 0;
+}
+template <class Sys, class Tab>
+constexpr bool lone_forward(bool adaptive)
+{
+    return Sys::N <= 4 && Sys::N * Tab::SF + Sys::P + stage_constants<Tab>(Tab::SF) +
+                                  (adaptive ? control_constants<Tab>() : 0) <=
+                              VA_LONE_DOUBLES;
+}
+// replay: an observed reverse, which runs the forward's steps again
+template <class Sys, class Tab, int NS>
+constexpr bool lone_reverse(bool replay = false)
+{
+    return Sys::N <= 4 && (1 + NS) * (Sys::N * Tab::S + Sys::P) + stage_constants<Tab>(Tab::S) +
+                                  (replay ? control_constants<Tab>() : 0) <=
+                              VA_LONE_DOUBLES;
 }
 
 template <class Sys, class Tab, bool Ad>
 struct Launch {
     static hipError_t fwd(const FwdArgs &a, int grid, int block, hipStream_t s)
     {
-        if constexpr (Sys::N <= 4) {
-            if (lone_waves<Sys>(grid, block)) {
+        if constexpr (lone_forward<Sys, Tab>(Ad)) {
+            if (lone_waves(grid, block)) {
                 hipLaunchKernelGGL((k_fwd<Sys, Tab, Ad, true>), dim3(grid), dim3(block), 0, s, a);
                 return hipGetLastError();
             }
@@ -765,29 +808,29 @@ struct Launch {
     }
     // two seeds through one sweep where the state leaves room for both
     static constexpr bool kSeedPairs = Sys::N <= 4 && Sys::P <= 8;
-    template <bool Lone>
+    template <int NS>
     static hipError_t rev_as(const RevArgs &a, int grid, int block, hipStream_t s)
     {
-        if constexpr (kSeedPairs) {
-            if (rev_items(a).per > 1) {
-                hipLaunchKernelGGL((k_rev<Sys, Tab, Lone, 2>), dim3(grid), dim3(block), 0, s, a);
+        if constexpr (lone_reverse<Sys, Tab, NS>()) {
+            if (lone_waves(grid, block)) {
+                hipLaunchKernelGGL((k_rev<Sys, Tab, true, NS>), dim3(grid), dim3(block), 0, s, a);
                 return hipGetLastError();
             }
         }
-        hipLaunchKernelGGL((k_rev<Sys, Tab, Lone, 1>), dim3(grid), dim3(block), 0, s, a);
-        return hipGetLastError();
-    }
-    static hipError_t rev(const RevArgs &a, int grid, int block, hipStream_t s)
-    {
-        if constexpr (Sys::N <= 4)
-            if (lone_waves<Sys>(grid, block)) return rev_as<true>(a, grid, block, s);
-        if constexpr (Sys::N == 2) {
+        if constexpr (Sys::N == 2 && NS == 1) {
             if (a.slot && rev_items(a).seeds == 1 && !a.identity) {
                 hipLaunchKernelGGL((k_rev_lines<Sys, Tab>), dim3(grid), dim3(block), 0, s, a);
                 return hipGetLastError();
             }
         }
-        return rev_as<false>(a, grid, block, s);
+        hipLaunchKernelGGL((k_rev<Sys, Tab, false, NS>), dim3(grid), dim3(block), 0, s, a);
+        return hipGetLastError();
+    }
+    static hipError_t rev(const RevArgs &a, int grid, int block, hipStream_t s)
+    {
+        if constexpr (kSeedPairs)
+            if (rev_items(a).per > 1) return rev_as<2>(a, grid, block, s);
+        return rev_as<1>(a, grid, block, s);
     }
     static hipError_t pfwd(const PlainFwdArgs &a, int grid, int block, hipStream_t s)
     {

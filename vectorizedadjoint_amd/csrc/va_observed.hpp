@@ -745,14 +745,14 @@ struct LaunchObs {
     }
     static hipError_t fwd(const ObsFwdArgs &a, int grid, int block, hipStream_t s)
     {
-        if constexpr (Sys::N <= 4)
-            if (lone_waves<Sys>(grid, block)) return fwd_as<true>(a, grid, block, s);
+        if constexpr (lone_forward<Sys, Tab>(true))
+            if (lone_waves(grid, block)) return fwd_as<true>(a, grid, block, s);
         return fwd_as<false>(a, grid, block, s);
     }
     static hipError_t rev(const ObsRevArgs &a, int grid, int block, hipStream_t s)
     {
-        if constexpr (Sys::N <= 4)
-            if (lone_waves<Sys>(grid, block)) return rev_as<true>(a, grid, block, s);
+        if constexpr (lone_reverse<Sys, Tab, 1>(true))
+            if (lone_waves(grid, block)) return rev_as<true>(a, grid, block, s);
         return rev_as<false>(a, grid, block, s);
     }
     // the smaller occupancy of the two storage variants, so one sizing serves both
