@@ -280,11 +280,14 @@ __global__ void __launch_bounds__(VA_ORDER_BUCKETS) k_order_hist(va::OrderArgs a
 // The instances in buckets >= va::OrderArgs::long_bucket, at most VA_LONG_MAX, are the
 // head of an order that the long-instance kernels take; their count goes to n_long.
 // For a forward that is 256 attempts and more, or, with a batch above 5/3 of the
-// lanes in flight, 448: the bulk beside the long instances then ends last, and the
-// long kernel's waves, one instance each, take more from it than the instances
-// do (GLV, t1=50, solve at 256 / 448: N=10, lanes 36864, B=48000 1.88 / 1.99 ms,
-// 58000 2.12 / 2.12, 65536 2.38 / 2.29, 80000 2.95 / 2.84; N=5, lanes 73728,
-// B=150000 4.47 / 4.38; N=16, lanes 24576, B=40000 5.44 / 5.50).
+// instances that the device holds in flight, 448: the bulk beside the long
+// instances then ends last, and the long kernel's waves, one instance each, take
+// more from it than the instances do.  Solves at 256 / 448 (N=10, the one size
+// with long-instance kernels; 36,864 in flight; Cash-Karp, tol 1e-8, t1=50 where not
+// stated): B=48000 1.88 / 1.99 ms, 58000 2.12 / 2.12, 65536 2.40 / 2.28, 80000
+// 2.91 / 2.82, 120000 4.19 / 4.17; B=65536 with DOPRI5 2.73 / 2.57, tol 1e-9
+// 3.01 / 2.90, and within the spread of a side (2%) with tol 1e-6, t1=15 and
+// Fehlberg 7(8).
 constexpr int VA_LONG_BUCKET = 32;       // 256 attempts (or accepted steps)
 constexpr int VA_LONG_BUCKET_FULL = 56;  // 448
 constexpr int VA_LONG_MAX = 256;    // one block each
@@ -404,6 +407,7 @@ struct va_handle {
     int cu_count = 0;
     int block = 256;
     int64_t lanes_fwd = 0, lanes_rev = 0;  // instances in flight of the persistent kernels
+    int64_t lanes_full = 0;                // and of a forward that fills the device
     // persistent store and its row layout; slot [B] is null where instance b is slot b
     double *traj = nullptr;
     va::RowLayout rows;
@@ -580,7 +584,7 @@ va_status build_orders(va_handle *h, int modes, bool next, const CountsOut &out,
     a.order[1] = next ? h->order_fwd_next : h->order_fwd;
     a.n_long[1] = h->counters + (next ? 11 - h->nlong_idx : h->nlong_idx);
     a.long_bucket[0] = VA_LONG_BUCKET;
-    a.long_bucket[1] = 3 * a.B > 5 * h->lanes_fwd ? VA_LONG_BUCKET_FULL : VA_LONG_BUCKET;
+    a.long_bucket[1] = 3 * a.B > 5 * h->lanes_full ? VA_LONG_BUCKET_FULL : VA_LONG_BUCKET;
     if (modes & 2) h->ordered = true;
     const int grid = blocks_for(a.B, VA_ORDER_BUCKETS * a.items);
     hipLaunchKernelGGL(k_order_hist, dim3(grid), dim3(VA_ORDER_BUCKETS), 0, s, a, out);
@@ -1232,13 +1236,15 @@ va_status create_handle(const va_problem *pb_in, const va::KernelSet *given, va_
         // shared-parameter tiles: one workgroup per CU (the matrix fills the LDS)
         const int64_t ntiles = (B + ks.shared_tile - 1) / ks.shared_tile;
         h->shared_grid = (int)std::min<int64_t>(ntiles, h->cu_count);
-    } else if (pb->lanes > 0) {
-        h->lanes_fwd = h->lanes_rev = pb->lanes;
     } else {
-        // every resident instance slot of the device
+        // every resident instance slot of the device, or as many as the caller says
         const int64_t per_block = ks.slots(h->block);
-        h->lanes_fwd = (int64_t)std::max(1, ks.occ_fwd(h->block)) * h->cu_count * per_block;
-        h->lanes_rev = (int64_t)std::max(1, ks.occ_rev(h->block)) * h->cu_count * per_block;
+        h->lanes_full = (int64_t)std::max(1, ks.occ_fwd(h->block)) * h->cu_count * per_block;
+        h->lanes_fwd = pb->lanes > 0 ? pb->lanes : h->lanes_full;
+        h->lanes_rev =
+            pb->lanes > 0
+                ? pb->lanes
+                : (int64_t)std::max(1, ks.occ_rev(h->block)) * h->cu_count * per_block;
     }
     const double budget = (double)pb->trajectory_budget_bytes;
     bool full_store = true;  // per-step rows in h->traj / h->ptraj
