@@ -1,0 +1,29 @@
+"""Which reverse kernel a Lotka-Volterra call takes, CPU only: the blocks of three waves
+for the head of the order (the HEAD instantiation with part 2) in one-seed reverses of
+up to 16 species, adaptive, in blocks of 256 threads, and nowhere else."""
+import pytest
+
+import launches as L
+from vectorizedadjoint_amd import constants as K
+
+
+@pytest.fixture(scope="module")
+def exe(tmp_path_factory):
+    return L.build(tmp_path_factory.mktemp("launches"))
+
+
+@pytest.mark.parametrize("n", range(2, 33))
+def test_head_blocks_of_one_seed_reverses(exe, n):
+    for tableau, adaptive in ((K.TAB_CASH_KARP54, 1), (K.TAB_DOPRI5, 1), (K.TAB_FEHLBERG78, 1),
+                              (K.TAB_RK4, 0)):
+        calls = L.log(exe, ["solve", "forward", "adjoint:1", "adjoint:2", "sens"],
+                      system=K.SYS_LOTKA_VOLTERRA, n=n, np=n + n * n, tableau=tableau,
+                      adaptive=adaptive, batch=600)
+        head = n <= 16 and adaptive
+        for op, call in zip(("solve", "forward", "adjoint:1", "adjoint:2", "sens"), calls):
+            revs = [l for l in call if l.kernel.startswith("k_glv_rows_rev<")]
+            assert len(revs) == (op != "forward"), (op, call)
+            for l in revs:
+                one = op in ("solve", "adjoint:1")
+                assert (l["part"] == "2") == (head and one), (op, l)
+                assert l["items"] == {"adjoint:2": "2", "sens": str(n)}.get(op, "1")
