@@ -27,3 +27,16 @@ def test_head_blocks_of_one_seed_reverses(exe, n):
                 one = op in ("solve", "adjoint:1")
                 assert (l["part"] == "2") == (head and one), (op, l)
                 assert l["items"] == {"adjoint:2": "2", "sens": str(n)}.get(op, "1")
+
+
+@pytest.mark.parametrize("n", (2, 5, 10, 13, 16, 17))
+def test_reverses_without_a_head_take_the_kernel_without_its_lds(exe, n):
+    system = dict(system=K.SYS_LOTKA_VOLTERRA, n=n, np=n + n * n, batch=600)
+    for tableau in (K.TAB_CASH_KARP54, K.TAB_DOPRI5, K.TAB_FEHLBERG78):
+        # few lanes: from the second solve on beside the long-instance kernel, for N=10
+        for lanes in (0, 30):
+            for call in L.log(exe, ["solve", "solve", "forward", "adjoint:1", "adjoint:2", "sens"],
+                              tableau=tableau, lanes=lanes, **system):
+                for l in call:
+                    if l.kernel.startswith("k_glv_rows_rev<"):
+                        assert l.kernel.endswith("true>") == (l["part"] == "2"), l
