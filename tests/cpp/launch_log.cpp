@@ -33,6 +33,7 @@ std::map<const void *, std::string> &names()
 std::map<char *, std::pair<size_t, int>> bufs;  // address -> size, number
 std::set<const void *> written;                 // orders that a launch that ran has written
 int n_bufs = 0, occupancy = 2;
+size_t in_use = 0;  // bytes by hipMalloc
 bool capturing = false, quiet = true;
 struct Call {
     dim3 grid, block;
@@ -157,10 +158,20 @@ hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, in
 }
 const char *hipGetErrorString(hipError_t) { return "error"; }
 hipError_t hipGetLastError() { return hipSuccess; }
-hipError_t hipMalloc(void **p, size_t n) { return *p = new_buf(n), hipSuccess; }
+hipError_t hipMalloc(void **p, size_t n)
+{
+    const char *most = getenv("LAUNCH_LOG_MEMORY");  // bytes of the device; unset: any
+    if (most && in_use + n > strtoull(most, nullptr, 10)) return hipErrorOutOfMemory;
+    in_use += n;
+    return *p = new_buf(n), hipSuccess;
+}
 hipError_t hipMallocAsync(void **p, size_t n, hipStream_t) { return *p = new_buf(n), hipSuccess; }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return *p = new_buf(n), hipSuccess; }
-hipError_t hipFree(void *) { return hipSuccess; }
+hipError_t hipFree(void *p)
+{
+    if (p) in_use -= bufs[(char *)p].first;
+    return hipSuccess;
+}
 hipError_t hipFreeAsync(void *, hipStream_t) { return hipSuccess; }
 hipError_t hipHostFree(void *) { return hipSuccess; }
 hipError_t hipMemset(void *, int, size_t) { return hipSuccess; }

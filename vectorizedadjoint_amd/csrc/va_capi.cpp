@@ -1378,18 +1378,18 @@ va_status create_handle(const va_problem *pb_in, const va::KernelSet *given, va_
                 h->rows = va::rows_tiled(pb->max_steps, F);
                 const size_t tiles = ((size_t)B + va::VA_ROW_TILE - 1) / va::VA_ROW_TILE;
                 const size_t bytes = sizeof(double) * tiles * (size_t)h->rows.tile;
-                if (budget > 0.0 &&
-                    (double)bytes + 4.0 * (double)B * ((double)pb->n_obs + 1.0) > budget) {
-                    tiled = false;
-                } else if (hipMalloc((void **)&h->traj, bytes) != hipSuccess) {
+                tiled = budget <= 0.0 ||
+                        (double)bytes + 4.0 * (double)B * ((double)pb->n_obs + 1.0) <= budget;
+                if (tiled && (hipMalloc((void **)&h->slot, sizeof(int32_t) * (size_t)B) != hipSuccess ||
+                              hipMalloc((void **)&h->traj, bytes) != hipSuccess)) {
                     (void)hipGetLastError();
+                    hipFree(h->slot);
+                    h->slot = nullptr;
                     h->traj = nullptr;
                     tiled = false;
                 }
             }
-            if (tiled) {
-                alloc((void **)&h->slot, sizeof(int32_t) * (size_t)B);
-            } else {
+            if (!tiled) {
                 h->rows = va::rows_instance_major(pb->max_steps, F);
                 alloc((void **)&h->traj, sizeof(double) * rows * (size_t)B * F);
             }
