@@ -1018,8 +1018,8 @@ constexpr int VA_SPIN_LIMIT = 1 << 22;   // polls of a ring counter (about 0.1 s
 // LDS a long-instance block reserves beyond its own use (17 KB for N=10, with
 // Fehlberg 7(8) 30 KB), so that no two such blocks share a CU's 160 KB: each long
 // forward then has a SIMD without another long wave (two long waves on one SIMD
-// each ran ~40% slower), and the persistent kernels' blocks (14 KB of a forward, 4
-// KB of a reverse without a head) still fit beside it.
+// each ran ~40% slower), and two of the persistent kernels' blocks (14 KB of a
+// forward, 16 KB of a reverse, with Fehlberg 7(8) 29 KB) still fit beside it.
 constexpr int VA_LONG_LDS_PAD = 68 * 1024;
 
 template <int NN, class Tab>
@@ -1282,10 +1282,7 @@ __device__ __forceinline__ void glv_long_accumulate(const RevArgs &a, int64_t b,
 // then joins the others, which take the rest of the order from the start.  The
 // longest chain of a reverse without a long-instance kernel beside it so takes
 // 0.5 us per step instead of 1.6 (N=10, B=20000, index order: reverse 1.5 -> 0.54 ms).
-// Head: the variant that can.  It has the ring in LDS (12 KB for N=10) and may need
-// more registers (N=2 with Fehlberg 7(8): 227 against 164, two blocks per CU
-// against three), so every other reverse is launched without (that system's two
-// seeds, B=200000: 1.23 -> 1.15 ms).
+// Head: the variant that can, with the ring in LDS (12 KB for N=10).
 template <int NN, class Tab, bool Head>
 __global__ void __launch_bounds__(256) k_glv_rows_rev(RevArgs a)
 {
@@ -1595,6 +1592,13 @@ template <int NN, class Tab, bool Ad, bool WithLong = true>
 struct LaunchGlvRows {
     // three-wave blocks for the reverse's long head, taken with part 2
     static constexpr bool kHead = Ad && rows_rev_head(NN);
+    // A head's staging wave with 13 stages takes some 230 registers.  Where the sweep
+    // itself stays below 168 that is a third block per CU lost, and reverses without a
+    // head are launched as the variant that has none (N=2, Fehlberg 7(8), 227 registers
+    // against 164; B=200000, two seeds 1.23 -> 1.15 ms).  Everywhere else both variants
+    // have the same blocks per CU, LDS included, and the one with a head serves all
+    // (headline solve 2.31 ms, with the other for its bulk 2.33).
+    static constexpr bool kLean = kHead && Tab::S > 7 && NN == 2;
     // The persistent forward with two rows per lane where N is even and small
     // enough for both rows' parameters to stay in registers, when the instances
     // come longest-first (a.order): a wave then holds instances of similar
@@ -1634,20 +1638,19 @@ struct LaunchGlvRows {
     }
     static hipError_t rev(const RevArgs &a, int grid, int block, hipStream_t s)
     {
-        if constexpr (kHead) {
-            if (a.split && a.part == 2) {
-                // in blocks of 256; the grid is sized for the variant without, so no block
-                // more than the 256 CUs hold of this one, whose groups would only find
-                // the queue empty (N=2, Fehlberg 7(8), B=200000, three blocks per CU
-                // where two fit: reverse 0.72 ms, so 0.68)
-                static const int held = 256 * resident<true>(256);
-                grid = std::min(grid, held);
-                hipLaunchKernelGGL((k_glv_rows_rev<NN, Tab, true>), dim3(grid), dim3(block), 0, s,
+        if constexpr (kLean) {
+            if (!a.split || a.part != 2) {
+                hipLaunchKernelGGL((k_glv_rows_rev<NN, Tab, false>), dim3(grid), dim3(block), 0, s,
                                    a);
                 return hipGetLastError();
             }
+            // no block more than the 256 CUs hold of the variant with a head, whose groups
+            // would only find the queue empty (three blocks per CU where two fit,
+            // B=200000: reverse 0.72 ms, so 0.68)
+            static const int held = 256 * resident<true>(256);
+            grid = std::min(grid, held);
         }
-        hipLaunchKernelGGL((k_glv_rows_rev<NN, Tab, false>), dim3(grid), dim3(block), 0, s, a);
+        hipLaunchKernelGGL((k_glv_rows_rev<NN, Tab, kHead>), dim3(grid), dim3(block), 0, s, a);
         return hipGetLastError();
     }
     static hipError_t lng(const FwdArgs &fa, const RevArgs &ra, int grid, int block,
@@ -1694,7 +1697,7 @@ struct LaunchGlvRows {
                 &nb, k_glv_rows_fwd<NN, Tab, Ad, Lay::Groups>, block, 0);
         return e == hipSuccess ? nb : 1;
     }
-    static int occ_rev(int block) { return resident<false>(block); }
+    static int occ_rev(int block) { return resident<kHead && !kLean>(block); }
     // blocks of the reverse on a CU
     template <bool Head>
     static int resident(int block)
