@@ -46,7 +46,7 @@ struct FwdArgs {
     SolveParams sp;
     double *y;             // [N][B] in y0, out y(T)
     const double *p;       // [P][B]; Lotka-Volterra persistent kernels: [B][P]
-    double *traj;          // [B][cap+1][N+1] rows (t, y)
+    double *traj;          // rows (t, h, y), instance-major [B][cap+1][N+2] or as `rows` says
     int32_t *n_acc, *n_rej, *status;
     int32_t *counter;
     int32_t *max_steps_seen;
@@ -144,7 +144,7 @@ struct PlainRevArgs {
 // trajectory either stored in full or kept as checkpoints.
 struct ObsStore {
     int32_t ckpt;          // 0: full rows (t, h, y) in traj; 1: checkpoints in ck
-    double *traj;          // [B][cap+1][N+2]
+    double *traj;          // rows (t, h, y), placed by `rows`
     double *ck;            // [B][slots][N+3] (t, dt to try, observations taken, y)
     int32_t slots;         // checkpoints per instance (even)
     int32_t stride_max;    // largest checkpoint spacing; slots * stride_max >= cap

@@ -62,7 +62,7 @@ VA_POW_HD double from_halves(uint32_t hi, uint32_t lo)
 
 // The algorithm's constants, as literals: each use forms the 64-bit value in a
 // scalar register pair.  A caller may pass an object with the same members
-// instead (CtrlRegs in va_device.hpp keeps them in vector registers).
+// instead (PowRegs in va_device.hpp keeps them in vector registers).
 struct PowLiterals {
     // log1p polynomial, scaled by the evaluation (p0 = -1/2)
     static constexpr double P0 = -0x1p-1;
