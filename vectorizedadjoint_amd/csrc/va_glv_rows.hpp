@@ -1611,7 +1611,21 @@ struct LaunchGlvRows {
     // of any size where a wave of the Groups layout would hold no more than six
     // instances.  (Forward of N=10, B=4096, chains of 1,500 attempts: 2.23 -> 1.81
     // ms; B=20000 2.57 -> 2.13 ms; B=65536, a first solve, 4.2 -> 3.6 ms.)
+    //
+    // With two to four species a wave of the Groups layout holds 16 to 32 instances,
+    // and its exchanges cost less than the waves that Rows has more of (Cash-Karp,
+    // t1=10, Groups / Rows: N=2 B=256 80 / 95 us, 8000 146 / 244; N=3 1000 82 / 74,
+    // 2000 89 / 99, 8000 174 / 240; N=4 1000 84 / 77, 2000 99 / 101, 8000 196 / 248).
+    // From N=5 on that is so only without a blow-up in the batch, which Rows ends
+    // sooner (N=5 B=8192 214 / 254 us without; with one, forward and five seeds 1.44 /
+    // 1.26 ms).  Fixed steps have
+    // no long chains: Rows to one wave per SIMD (RK4, N=5 4000 256 / 235, 8000 270 /
+    // 313; N=10 4000 353 / 317, 8000 441 / 467, in index order 20000 759 / 1018).
     static constexpr int kRowsWaves = 256 * 4 * 2;
+    static constexpr int kRowsBatch = NN <= 2   ? 0
+                                      : !Ad     ? 2 * kRowsWaves
+                                      : NN >= 5 ? 4 * kRowsWaves
+                                                : kRowsWaves / 2;
     static hipError_t fwd(const FwdArgs &a, int grid, int block, hipStream_t s)
     {
         if constexpr (kPairs) {
@@ -1621,8 +1635,8 @@ struct LaunchGlvRows {
                 return hipGetLastError();
             }
         }
-        if constexpr (NN <= 16) {
-            if (a.sp.B <= 4 * kRowsWaves || (NN >= 10 && !a.order)) {
+        if constexpr (NN > 2 && NN <= 16) {
+            if (a.sp.B <= kRowsBatch || (Ad && NN >= 10 && !a.order)) {
                 const int64_t instances = std::min<int64_t>((int64_t)grid * slots(block), a.sp.B);
                 const int64_t waves = std::min<int64_t>((instances + 3) / 4, kRowsWaves);
                 const int per_block = block / 64;
