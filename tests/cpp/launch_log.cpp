@@ -92,7 +92,8 @@ void log_launch(const void *f, dim3 g, dim3 b, void **args)
     } else if (starts(n, "k_rev") || starts(n, "k_glv_rows")) {
         const auto &a = *(const va::RevArgs *)args[0];
         order_read(a.order);
-        printf(" part=%d items=%d", a.split ? a.part : -1, va::rev_items(a).parts);
+        printf(" part=%d items=%d in_turn=%d", a.split ? a.part : -1, va::rev_items(a).parts,
+               a.in_turn != nullptr);
     } else if (starts(n, "k_obs_fwd")) {
         order_read(((const va::ObsFwdArgs *)args[0])->order);
     } else if (starts(n, "k_obs_rev")) {

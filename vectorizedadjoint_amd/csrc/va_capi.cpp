@@ -829,6 +829,29 @@ int32_t seeds_per_item(const va_handle *h, int nout)
     return h->pb.batch * nout <= (int64_t)h->cu_count * 4 * 64 ? 1 : 2;
 }
 
+// A large batch of few species fills the chip with one seed, and a short sweep finds
+// its rows in the caches from the second seed on, so there the groups take the seeds
+// in turn (RevArgs::in_turn), unless the forward had instances of 256 and more
+// accepted steps, whose chains would follow one another, or the seeds of up to six
+// instances fill a wave, which then reads each row once for all of them.  Cash-Karp,
+// t1=10, B=64000, two, three and five seeds in turn / as items, ms: N=2 0.30 / 0.42,
+// 0.35 / 0.62, 0.45 / 0.86; N=3 0.44 / 0.60, 0.52 / 0.67, 0.66 / 1.18; N=4 0.51 /
+// 0.64, 0.57 / 0.95, 0.74 / 1.41; N=5 0.73 / 0.72, 0.90 / 0.80, 1.33 / 1.72; N=6 0.72 /
+// 0.77, 0.87 / 1.29, 1.34 / 1.16; N=7 0.79 / 1.03, 1.06 / 0.98, 1.66 / 2.11; N=8 1.02 /
+// 0.93, 1.35 / 1.64, 2.18 / 2.49; B=24000, N=2 0.16 / 0.18, 0.21 / 0.23, 0.33 / 0.31,
+// N=5 0.35 / 0.33, 0.44 / 0.36, 0.63 / 0.57; with long instances, N=5 B=64000, t1=40,
+// 1.24 / 0.85, 1.75 / 0.93, 2.87 / 1.84.
+constexpr int64_t VA_IN_TURN_MIN = 32768;
+constexpr int VA_IN_TURN_SPECIES = 7;
+
+bool seeds_in_turn(const va_handle *h, int nout)
+{
+    if (h->ks.layout != 1 || h->ks.n > VA_IN_TURN_SPECIES || h->pb.batch <= VA_IN_TURN_MIN)
+        return false;
+    const int groups = h->ks.slots(64);  // instances of a wave
+    return groups % nout != 0 || groups / nout > 6;
+}
+
 // identity: the seeds are the unit vectors (lambda is not used, mu = 0.0 + sum).
 // same_call: the forward of this call precedes it on s (its counters are clear and
 // h->pim holds p).
@@ -889,6 +912,7 @@ va_status reverse_persistent(va_handle *h, const double *p, int cost, const doub
         a.split = h->counters + VA_REV_LONG;
         a.part = 2;
     }
+    if (parts > 1 && seeds_in_turn(h, nseed)) a.in_turn = h->counters + VA_REV_LONG;
     const int64_t lanes = std::min<int64_t>(h->lanes_rev, B * parts);
     VA_HIP(h->ks.rev(a, blocks_for(lanes, h->ks.slots(h->block)), h->block, s));
     if (im) return pbar_to_mu(h, mu, nseed, add, s);

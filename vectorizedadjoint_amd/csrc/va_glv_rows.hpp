@@ -786,6 +786,11 @@ __global__ void __launch_bounds__(256) k_glv_rows2_fwd(FwdArgs a)
 // instance (or of a further seed) only recomputes.  Every value is formed by
 // the same operations in the same order as in the oracle.
 // ---------------------------------------------------------------------------
+__device__ __forceinline__ bool seeds_in_turn(const RevArgs &a)
+{
+    return a.in_turn && *a.in_turn == 0;
+}
+
 template <int NN, class Tab, bool OneShot>
 __device__ __forceinline__ void glv_rows_rev_body(const RevArgs &a, int64_t one, int32_t one_seed)
 {
@@ -822,7 +827,11 @@ __device__ __forceinline__ void glv_rows_rev_body(const RevArgs &a, int64_t one,
     const double *rows = nullptr;
     double v[NN];
     const QueueRange q = queue_range(B, a.split, a.part);
-    const RevItems items = rev_items(a);
+    RevItems items = rev_items(a);
+    if (!OneShot && seeds_in_turn(a)) {
+        items.per = items.seeds;
+        items.parts = 1;
+    }
     // the seed o of the instance: its lambda, cleared sums, its last row
     auto start_sweep = [&]() {
         if (!a.cost)
@@ -1286,6 +1295,10 @@ __device__ __forceinline__ void glv_long_accumulate(const RevArgs &a, int64_t b,
 template <int NN, class Tab, bool Head>
 __global__ void __launch_bounds__(256) k_glv_rows_rev(RevArgs a)
 {
+    // the grid is for items of one seed each
+    if (seeds_in_turn(a) &&
+        (int64_t)blockIdx.x * (blockDim.x >> 6) * GlvRows<NN>::GPW >= a.sp.B)
+        return;
     if constexpr (Head) {
         __shared__ StageRing<NN, Tab> ring;
         if ((int)blockIdx.x < head_blocks(a.split, a.part)) {

@@ -90,6 +90,9 @@ struct RevArgs {
     int32_t identity = 0;
     RowLayout rows;                  // one-lane kernels
     const int32_t *slot = nullptr;   // [B] or null
+    // (Lotka-Volterra row kernels, several seeds) null, or a count of long instances:
+    // where it is 0 an item is an instance with all of its seeds after all
+    const int32_t *in_turn = nullptr;
 };
 
 // The work items of a reverse: groups of seeds per instance.
